@@ -1207,18 +1207,26 @@ k_pairs(double* __restrict__ F, double* __restrict__ partials,
         one(j, Rs4[j]);
       }
     } else {
-      int k = sub;
-      for (; k + 2 * TPA < n; k += 3 * TPA) {
-        int j0 = nbr[nb_at(k, i, Npad)], j1 = nbr[nb_at(k + TPA, i, Npad)], j2 = nbr[nb_at(k + 2 * TPA, i, Npad)];
+      // three entries per step; in a lane's last step the atom itself stands
+      // in for the entries past its end, whose terms are not evaluated, so
+      // that the end costs one round of loads and not one per entry
+      for (int k = sub; k < n; k += 3 * TPA) {
+        const bool on1 = k + TPA < n, on2 = k + 2 * TPA < n;
+        int j0 = nbr[nb_at(k, i, Npad)], j1 = i, j2 = i;
+        if (on1) j1 = nbr[nb_at(k + TPA, i, Npad)];
+        if (on2) j2 = nbr[nb_at(k + 2 * TPA, i, Npad)];
         double4 r0 = Rs4[j0], r1 = Rs4[j1], r2 = Rs4[j2];
         if (LJ == 2) {
           const double q0 = charge[j0], q1 = charge[j1], q2 = charge[j2];
-          one(j0, r0, q0, true); one(j1, r1, q1, true); one(j2, r2, q2, true);
+          one(j0, r0, q0, true);
+          if (on1) one(j1, r1, q1, true);
+          if (on2) one(j2, r2, q2, true);
         } else {
-          one(j0, r0); one(j1, r1); one(j2, r2);
+          one(j0, r0);
+          if (on1) one(j1, r1);
+          if (on2) one(j2, r2);
         }
       }
-      for (; k < n; k += TPA) { int j = nbr[nb_at(k, i, Npad)]; one(j, Rs4[j]); }
     }
   }
   if (TPA > 1) {
@@ -1449,21 +1457,21 @@ k_pairs_mx(double* __restrict__ F, double* __restrict__ partials, const int4* __
       }
       flush(a);
     } else {
-      int k = sub;
-      for (; k + 3 * TPA < n; k += 4 * TPA) {
-        int j0 = nbr[nb_at(k, i, Npad)], j1 = nbr[nb_at(k + TPA, i, Npad)];
-        int j2 = nbr[nb_at(k + 2 * TPA, i, Npad)], j3 = nbr[nb_at(k + 3 * TPA, i, Npad)];
+      // four entries per step, one FP32 sum each; a lane's last step as in k_pairs
+      for (int k = sub; k < n; k += 4 * TPA) {
+        const bool on1 = k + TPA < n, on2 = k + 2 * TPA < n, on3 = k + 3 * TPA < n;
+        int j0 = nbr[nb_at(k, i, Npad)], j1 = i, j2 = i, j3 = i;
+        if (on1) j1 = nbr[nb_at(k + TPA, i, Npad)];
+        if (on2) j2 = nbr[nb_at(k + 2 * TPA, i, Npad)];
+        if (on3) j3 = nbr[nb_at(k + 3 * TPA, i, Npad)];
         int4 q0 = Q4[j0], q1 = Q4[j1], q2 = Q4[j2], q3 = Q4[j3];
         MixedAcc a = { 0, 0, 0, 0, 0, 0, 0 };
-        one(j0, q0, a); one(j1, q1, a); one(j2, q2, a); one(j3, q3, a);
+        one(j0, q0, a);
+        if (on1) one(j1, q1, a);
+        if (on2) one(j2, q2, a);
+        if (on3) one(j3, q3, a);
         flush(a);
       }
-      MixedAcc a = { 0, 0, 0, 0, 0, 0, 0 };
-      for (; k < n; k += TPA) {
-        int j = nbr[nb_at(k, i, Npad)];
-        one(j, Q4[j], a);
-      }
-      flush(a);
     }
   }
   if (TPA > 1) {
@@ -1813,7 +1821,8 @@ Device* dev_create(const DeviceSetup& s) {
   HIP_CHECK(hipHostGetDevicePointer((void**)&d->hseqDev, d->hseq, 0));
   *d->hseq = 0;
   d->result.alloc(64);
-  d->partials.alloc(64 * (size_t)(Np / BLOCK + 1));   // up to 16 threads per atom x 4 sums
+  // four sums per block: up to 64 threads per atom for small systems, else 16
+  d->partials.alloc((s.N <= 16384 ? 256 : 64) * (size_t)(Np / BLOCK + 1));
   d->trigPart.alloc(2 * (size_t)(Np / BLOCK + 1));
   d->trig.alloc(4);
   HIP_CHECK(hipMemsetAsync(d->Rs4.p, 0, sizeof(double4) * Np, d->stream));
@@ -2248,7 +2257,7 @@ void dev_compute_pairs(Device* d, const PairCall& c, ForceSums* out) {
   hipEvent_t e0 = d->profiling ? d->ev0 : nullptr, e1 = d->profiling ? d->ev1 : nullptr;
   bool U = c.ntypes == 1;
   bool LJ = lj_path(d, c.layer);
-  // threads per atom: enough wavefronts to fill the chip (at least 2^18
+  // threads per atom, 1, 4, 16, 32 or 64: enough wavefronts to fill the chip (at least 2^18
   // lanes) and about 24 list entries per lane, so that long lists (water at
   // rc 10 A holds ~700 entries per atom) are spread over many waves
   int tpa = 1;
@@ -2256,10 +2265,20 @@ void dev_compute_pairs(Device* d, const PairCall& c, ForceSums* out) {
     long lanes = std::max(1L << 18, (long)(d->listEntries / 24.0));
     long want = lanes / std::max(N, 1);
     tpa = want >= 16 ? 16 : (want >= 4 ? 4 : 1);
+    // small systems with long lists go further, where 16 lanes leave SIMDs
+    // without a wave: a wave per atom up to 4,096 atoms with at least 96
+    // entries (3,000 water atoms, 726 entries: 40 -> 23 us; 800 LJ atoms, 120
+    // entries: step 52 -> 49 us; 4,000 LJ atoms with 75 entries: 60 -> 63 us,
+    // so they keep 16), 32 lanes up to 16,384 atoms with at least 384
+    // (12,288 water atoms: step 315 -> 311 us; 98,304: 598 -> 612 us)
+    const double each = d->listEntries / std::max(N, 1);
+    if (N <= 4096 && want >= 64 && each >= 96.0) tpa = 64;
+    else if (N <= 16384 && want >= 24 && each >= 384.0) tpa = 32;
   }
   int gp = div_up((long)N * tpa, BLOCK);
   // the pair kernels write four sums per block into partials, which holds
-  // 64 (Npad / BLOCK + 1) values: enough for up to 16 lanes per atom
+  // 64 (Npad / BLOCK + 1) values: enough for up to 16 lanes per atom (256
+  // and 64 lanes up to 16,384 atoms)
   if ((size_t)gp * 4 > d->partials.n) fatal("compute_forces", "too many lanes per atom for the partial sums");
   double* ea = d->wantAtomE ? d->eatom.p : nullptr;
   int variant = (c.energy ? 4 : 0) + (U ? 2 : 0) + (LJ ? 1 : 0);
@@ -2283,7 +2302,8 @@ void dev_compute_pairs(Device* d, const PairCall& c, ForceSums* out) {
                         Np, ea, ljt, ljk)
 #define GENERIC_MX_J(E, U, J)                                                                                      \
   do {                                                                                                            \
-    if (tpa == 16) LAUNCH_MX(E, U, J, 16); else if (tpa == 4) LAUNCH_MX(E, U, J, 4);                              \
+    if (tpa == 64) LAUNCH_MX(E, U, J, 64); else if (tpa == 32) LAUNCH_MX(E, U, J, 32);                            \
+    else if (tpa == 16) LAUNCH_MX(E, U, J, 16); else if (tpa == 4) LAUNCH_MX(E, U, J, 4);                         \
     else LAUNCH_MX(E, U, J, 1);                                                                                   \
   } while (0)
 #define GENERIC_MX(E, U)                                                                                           \
@@ -2312,7 +2332,8 @@ void dev_compute_pairs(Device* d, const PairCall& c, ForceSums* out) {
                         c.Rc2, N, Np, ea, ljt, ljk)
 #define GENERIC_J(E, U, J)                                                                                         \
   do {                                                                                                            \
-    if (tpa == 16) LAUNCH_PAIRS(E, U, J, 16); else if (tpa == 4) LAUNCH_PAIRS(E, U, J, 4);                        \
+    if (tpa == 64) LAUNCH_PAIRS(E, U, J, 64); else if (tpa == 32) LAUNCH_PAIRS(E, U, J, 32);                      \
+    else if (tpa == 16) LAUNCH_PAIRS(E, U, J, 16); else if (tpa == 4) LAUNCH_PAIRS(E, U, J, 4);                   \
     else LAUNCH_PAIRS(E, U, J, 1);                                                                                \
   } while (0)
 #define GENERIC(E, U)                                                                                              \
