@@ -138,6 +138,7 @@ EwaldHost ewald_initialize(double accuracy, double Rc, double L, int nlayers, co
 
   // k-vectors: kspace_ewald.f90:103-184
   double unit = 2.0 * PI_ / L, unitSq = unit * unit;
+  e.unit = unit;
   int nmax = (int)std::ceil(h.kmax / unit);
   int M = 2 * nmax + 1, maxnvecs = M * M * M / 2, M2M3 = M * M;
   double kmaxSq = unitSq * nmax * nmax;
@@ -184,6 +185,7 @@ EwaldSetup lowk_setup(const EwaldSetup& full, int layer, double alpha, double L,
   int nt = full.nt;
   e.lambda.assign(full.lambda.begin() + (size_t)(layer - 1) * nt * nt, full.lambda.begin() + (size_t)layer * nt * nt);
   double unit = 2.0 * PI_ / L, unitSq = unit * unit, kcutSq = kcut * kcut;
+  e.unit = unit;
   int nmax = std::max(1, (int)std::ceil(kcut / unit));
   std::vector<int> n;
   for (int n1 = 0; n1 <= nmax; n1++)
