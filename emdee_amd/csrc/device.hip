@@ -62,7 +62,10 @@ static void post_wait(Device* d, unsigned long long seq) {
 }
 
 void dev_post_wait(Device* d, unsigned long long seq) { post_wait(d, seq); }
-void dev_wait_posts(Device* d) { post_wait(d, d->seq); }
+void dev_wait_posts(Device* d) {
+  dev_flush_pairs(d);
+  post_wait(d, d->seq);
+}
 
 __global__ void k_iota(int* p, int n) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -164,10 +167,55 @@ __device__ __forceinline__ double disp_sq(const double* __restrict__ R, const do
   return dx * dx + dy * dy + dz * dz;
 }
 
+// (max, first index) of a set of pairs: the larger value wins, ties go to the
+// smaller index, so any combination order gives the same pair.
+__device__ __forceinline__ void max_first(double& v, double& idx, double ov, double oi) {
+  if (ov > v || (ov == v && oi < idx)) { v = ov; idx = oi; }
+}
+// Reduces nb blocks' {max, first index} into trig and posts them to the host
+// (as k_reduce_post); one block.
+__device__ __forceinline__ void trig_post(double* __restrict__ trig, const double* __restrict__ part, int nb,
+                                          double* __restrict__ host, unsigned long long* __restrict__ hostSeq,
+                                          unsigned long long seq) {
+  __shared__ double smax[BLOCK / 64], sidx[BLOCK / 64];
+  double v = -1.0, idx = 2147483647.0;
+#pragma unroll 8
+  for (int b = threadIdx.x; b < nb; b += BLOCK) max_first(v, idx, part[2 * b], part[2 * b + 1]);
+  for (int off = 32; off > 0; off >>= 1) max_first(v, idx, __shfl_down(v, off, 64), __shfl_down(idx, off, 64));
+  int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (lane == 0) { smax[w] = v; sidx[w] = idx; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < BLOCK / 64; k++) max_first(v, idx, smax[k], sidx[k]);
+    trig[0] = v;
+    trig[1] = idx;
+    host[0] = v;
+    host[1] = idx;
+    __threadfence_system();
+    *(volatile unsigned long long*)hostSeq = seq;
+  }
+}
+__global__ void k_disp_a_reduce(double* __restrict__ trig, const double* __restrict__ part, int nb,
+                                double* __restrict__ host, unsigned long long* __restrict__ hostSeq,
+                                unsigned long long seq) {
+  trig_post(trig, part, nb, host, hostSeq, seq);
+}
+// Thread 0's {max, first index} of a block of pass A: left in part, and posted
+// by the last block when the grid finishes it (finish_sums)
+__device__ __forceinline__ void finish_trig(const Post& post, double* __restrict__ trig, double* __restrict__ part,
+                                            double v, int idx) {
+  if (threadIdx.x == 0) {
+    part[2 * blockIdx.x] = v;
+    part[2 * blockIdx.x + 1] = (double)idx;
+  }
+  if (post.ticket && last_block(post.ticket, gridDim.x))
+    trig_post(trig, part, gridDim.x, post.host, post.hostSeq, post.seq);
+}
 // Pass A also writes the scaled positions of the current coordinates (sc),
 // which the pair kernels of the same force evaluation read.
 __global__ void k_disp_a(double* __restrict__ part, const double* __restrict__ R, const double* __restrict__ R0,
-                         const int* __restrict__ perm, int N, int Npad, Scaled sc) {
+                         const int* __restrict__ perm, int N, int Npad, Scaled sc, double* __restrict__ trig,
+                         Post post) {
   __shared__ double smax[BLOCK / 64];
   __shared__ int sidx[BLOCK / 64];
   int s = blockIdx.x * BLOCK + threadIdx.x;
@@ -189,36 +237,8 @@ __global__ void k_disp_a(double* __restrict__ part, const double* __restrict__ R
   if (threadIdx.x == 0) {
     for (int w = 1; w < BLOCK / 64; w++)
       if (smax[w] > v || (smax[w] == v && sidx[w] < idx)) { v = smax[w]; idx = sidx[w]; }
-    part[2 * blockIdx.x] = v;
-    part[2 * blockIdx.x + 1] = (double)idx;
   }
-}
-// (max, first index) of a set of pairs: the larger value wins, ties go to the
-// smaller index, so any combination order gives the same pair.
-__device__ __forceinline__ void max_first(double& v, double& idx, double ov, double oi) {
-  if (ov > v || (ov == v && oi < idx)) { v = ov; idx = oi; }
-}
-// ... and posts {max, first index} to the host as well (as k_reduce_post)
-__global__ void k_disp_a_reduce(double* __restrict__ trig, const double* __restrict__ part, int nb,
-                                double* __restrict__ host, unsigned long long* __restrict__ hostSeq,
-                                unsigned long long seq) {
-  __shared__ double smax[BLOCK / 64], sidx[BLOCK / 64];
-  double v = -1.0, idx = 2147483647.0;
-#pragma unroll 8
-  for (int b = threadIdx.x; b < nb; b += BLOCK) max_first(v, idx, part[2 * b], part[2 * b + 1]);
-  for (int off = 32; off > 0; off >>= 1) max_first(v, idx, __shfl_down(v, off, 64), __shfl_down(idx, off, 64));
-  int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (lane == 0) { smax[w] = v; sidx[w] = idx; }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int k = 1; k < BLOCK / 64; k++) max_first(v, idx, smax[k], sidx[k]);
-    trig[0] = v;
-    trig[1] = idx;
-    host[0] = v;
-    host[1] = idx;
-    __threadfence_system();
-    *(volatile unsigned long long*)hostSeq = seq;
-  }
+  finish_trig(post, trig, part, v, idx);
 }
 __global__ void k_disp_c(double* __restrict__ part, const double* __restrict__ R, const double* __restrict__ R0,
                          const int* __restrict__ perm, const double* __restrict__ trig, int N, int Npad) {
@@ -1505,7 +1525,7 @@ k_pairs_mx(double* __restrict__ F, double* __restrict__ partials, const int4* __
 template <bool KE>
 __global__ void k_boost(double* __restrict__ P, double* __restrict__ partials, const double* __restrict__ F,
                         const double* __restrict__ invMass, const int* __restrict__ freeFlag,
-                        double CP, double CF, int translate, int N, int Npad) {
+                        double CP, double CF, int translate, int N, int Npad, Post post) {
   int blk = blockIdx.x;
   int s = blk * BLOCK + threadIdx.x;
   double v[3] = { 0, 0, 0 };
@@ -1520,14 +1540,14 @@ __global__ void k_boost(double* __restrict__ P, double* __restrict__ partials, c
   }
   if (KE) {
     block_sum<3>(v);
-    if (threadIdx.x == 0) { partials[3 * blk] = v[0]; partials[3 * blk + 1] = v[1]; partials[3 * blk + 2] = v[2]; }
+    finish_sums<3>(post, partials, v, blk);
   }
 }
 // The same kick for free atoms of one mass, two neighbouring slots per
 // thread (16-byte loads and stores; the second slot is left alone past N).
 template <bool KE>
 __global__ void k_boost_u2(double* __restrict__ P, double* __restrict__ partials, const double* __restrict__ F,
-                           double CP, double CF, int translate, int N, int Npad, double im) {
+                           double CP, double CF, int translate, int N, int Npad, double im, Post post) {
   int blk = blockIdx.x;
   int s = 2 * (blk * BLOCK + threadIdx.x);
   double v[3] = { 0, 0, 0 };
@@ -1548,7 +1568,7 @@ __global__ void k_boost_u2(double* __restrict__ P, double* __restrict__ partials
   }
   if (KE) {
     block_sum<3>(v);
-    if (threadIdx.x == 0) { partials[3 * blk] = v[0]; partials[3 * blk + 1] = v[1]; partials[3 * blk + 2] = v[2]; }
+    finish_sums<3>(post, partials, v, blk);
   }
 }
 // move, EmDeeData.f90:823-860 (free atoms): R = CR*R + CP*P*invMass.
@@ -1582,7 +1602,8 @@ __global__ void k_displace_u2(double* __restrict__ R, const double* __restrict__
 // thread: part holds one (max, index) pair per block of 2 BLOCK slots.
 __global__ void k_displace_u2_trig(double* __restrict__ R, const double* __restrict__ P, double CR, double CP,
                                    int N, int Npad, double im, const double* __restrict__ R0,
-                                   const int* __restrict__ perm, double* __restrict__ part, Scaled sc) {
+                                   const int* __restrict__ perm, double* __restrict__ part, Scaled sc,
+                                   double* __restrict__ trig, Post post) {
   __shared__ double smax[BLOCK / 64];
   __shared__ int sidx[BLOCK / 64];
   int s = 2 * (blockIdx.x * BLOCK + threadIdx.x);
@@ -1627,9 +1648,8 @@ __global__ void k_displace_u2_trig(double* __restrict__ R, const double* __restr
   if (threadIdx.x == 0) {
     for (int w = 1; w < BLOCK / 64; w++)
       if (smax[w] > v || (smax[w] == v && sidx[w] < idx)) { v = smax[w]; idx = sidx[w]; }
-    part[2 * blockIdx.x] = v;
-    part[2 * blockIdx.x + 1] = (double)idx;
   }
+  finish_trig(post, trig, part, v, idx);
 }
 
 // ---- shadow terms of EmDee_verlet_step, free atoms (EmDeeCode.f90:1167-1204)
@@ -1822,9 +1842,14 @@ Device* dev_create(const DeviceSetup& s) {
   *d->hseq = 0;
   d->result.alloc(64);
   // four sums per block: up to 64 threads per atom for small systems, else 16
-  d->partials.alloc((s.N <= 16384 ? 256 : 64) * (size_t)(Np / BLOCK + 1));
+  const size_t base = 16 * (size_t)(Np / BLOCK + 1);   // one count per block of a 16-lane list build
+  d->pairPartSize = (s.N <= 16384 ? 256 : 64) * (size_t)(Np / BLOCK + 1);
+  d->partials.alloc(base + d->pairPartSize);
+  d->pairPart = d->partials.p + base;
   d->trigPart.alloc(2 * (size_t)(Np / BLOCK + 1));
-  d->trig.alloc(4);
+  d->trig.alloc(4 + TICKETS);
+  d->tickets = reinterpret_cast<unsigned int*>(d->trig.p + 4);
+  HIP_CHECK(hipMemsetAsync(d->trig.p, 0, sizeof(double) * (4 + TICKETS), d->stream));
   HIP_CHECK(hipMemsetAsync(d->Rs4.p, 0, sizeof(double4) * Np, d->stream));
   d->key.alloc(Np); d->order.alloc(Np); d->nnb.alloc(Np); d->flags.alloc(4);
   HIP_CHECK(hipMemsetAsync(d->R.p, 0, 3 * sizeof(double) * Np, d->stream));
@@ -2027,22 +2052,28 @@ void dev_trigger_launch(Device* d, double L, bool mixed, int layer) {
   // test divides R by L itself)
   bool needRs4 = !mixed || !lj_path(d, layer);
   // (the FP32 charges change only with the slot order: the list build writes them)
+  d->trigSeq = 0;
   int nb = g;
   if (d->trigPreAt == d->posWrites && d->trigPreL == L && d->trigPreMixed == mixed && d->trigPreRs4 == needRs4) {
     nb = d->trigPreBlocks;               // the drift formed pass A for these positions
+    d->trigSeq = d->trigPreSeq;          // ... and posted it, on a small grid
   } else {
     Scaled sc{ needRs4 ? d->Rs4.p : nullptr, mixed ? d->Q4.p : nullptr, nullptr, d->type.p, d->charge.p,
                d->chargedFlag.p, L };
+    const Post post = dev_post(d, POST_TRIG, TICKET_TRIG, g, false);
     hipLaunchKernelGGL(k_disp_a, dim3(g), dim3(BLOCK), 0, d->stream, d->trigPart.p, d->R.p, d->R0.p, d->perm.p, N,
-                       d->Npad, sc);
+                       d->Npad, sc, d->trig.p, post);
+    if (post.ticket) d->trigSeq = post.seq;
   }
   d->trigKnown = true;
   d->trigMixed = mixed;
   d->trigRs4 = needRs4;
   d->trigL = L;
-  d->trigSeq = ++d->seq;
-  hipLaunchKernelGGL(k_disp_a_reduce, dim3(1), dim3(BLOCK), 0, d->stream, d->trig.p, d->trigPart.p, nb, d->hpostDev,
-                     d->hseqDev, d->trigSeq);
+  if (!d->trigSeq) {
+    d->trigSeq = ++d->seq;
+    hipLaunchKernelGGL(k_disp_a_reduce, dim3(1), dim3(BLOCK), 0, d->stream, d->trig.p, d->trigPart.p, nb,
+                       d->hpostDev + POST_TRIG, d->hseqDev, d->trigSeq);
+  }
   launch_check("trigger");
 }
 
@@ -2053,23 +2084,24 @@ void dev_trigger_launch(Device* d, double L, bool mixed, int layer) {
 bool dev_trigger_result(Device* d, double skinSq) {
   if (d->N == 0) return false;
   post_wait(d, d->trigSeq);
-  double maximum = d->hpost[0], approach;
+  const double* h = d->hpost + POST_TRIG;
+  double maximum = h[0], approach;
   if (maximum > skinSq) {
     approach = maximum;                    // a lower bound, enough to decide
-  } else if (d->hpost[1] != 0.0 && 4.0 * maximum * (1.0 + 1e-12) < skinSq) {
+  } else if (h[1] != 0.0 && 4.0 * maximum * (1.0 + 1e-12) < skinSq) {
     approach = 4.0 * maximum;              // an upper bound, enough to decide
   } else {
     double next = maximum;
-    if (d->hpost[1] != 0.0) {              // pass C: max over atoms before the first maximum
+    if (h[1] != 0.0) {              // pass C: max over atoms before the first maximum
       int N = d->N, g = div_up(N, BLOCK);
       hipLaunchKernelGGL(k_disp_c, dim3(g), dim3(BLOCK), 0, d->stream, d->partials.p, d->R.p, d->R0.p, d->perm.p,
                          d->trig.p, N, d->Npad);
       unsigned long long seq = ++d->seq;
       hipLaunchKernelGGL(k_disp_c_reduce, dim3(1), dim3(BLOCK), 0, d->stream, d->trig.p, d->partials.p, g,
-                         d->hpostDev, d->hseqDev, seq);
+                         d->hpostDev + POST_TRIG, d->hseqDev, seq);
       launch_check("trigger");
       post_wait(d, seq);
-      next = d->hpost[2];
+      next = h[2];
     }
     approach = maximum + 2 * std::sqrt(maximum * next) + next;
   }
@@ -2276,10 +2308,10 @@ void dev_compute_pairs(Device* d, const PairCall& c, ForceSums* out) {
     else if (N <= 16384 && want >= 24 && each >= 384.0) tpa = 32;
   }
   int gp = div_up((long)N * tpa, BLOCK);
-  // the pair kernels write four sums per block into partials, which holds
+  // the pair kernels write four sums per block into pairPart, which holds
   // 64 (Npad / BLOCK + 1) values: enough for up to 16 lanes per atom (256
   // and 64 lanes up to 16,384 atoms)
-  if ((size_t)gp * 4 > d->partials.n) fatal("compute_forces", "too many lanes per atom for the partial sums");
+  if ((size_t)gp * 4 > d->pairPartSize) fatal("compute_forces", "too many lanes per atom for the partial sums");
   double* ea = d->wantAtomE ? d->eatom.p : nullptr;
   int variant = (c.energy ? 4 : 0) + (U ? 2 : 0) + (LJ ? 1 : 0);
   if (c.mixed) {
@@ -2297,7 +2329,7 @@ void dev_compute_pairs(Device* d, const PairCall& c, ForceSums* out) {
     const bool ljc = d->ljcOk[c.layer] != 0;
 #define LAUNCH_MX(E, U, J, T)                                                                                      \
   hipExtLaunchKernelGGL((k_pairs_mx<E, U, J, T>), dim3(gp), dim3(BLOCK), 0, d->stream, e0, e1, 0, F,                \
-                        d->partials.p, (const int4*)d->Q4.p, (const double*)d->R.p, (const double4*)d->Rs4.p,     \
+                        d->pairPart, (const int4*)d->Q4.p, (const double*)d->R.p, (const double4*)d->Rs4.p,     \
                         (const int*)d->nbr.p, (const int*)d->nnb.p, (const float*)d->qf.p, pt, cp, c.ntypes, mc, N, \
                         Np, ea, ljt, ljk)
 #define GENERIC_MX_J(E, U, J)                                                                                      \
@@ -2327,7 +2359,7 @@ void dev_compute_pairs(Device* d, const PairCall& c, ForceSums* out) {
     const bool ljc = d->ljcOk[c.layer] != 0;
 #define LAUNCH_PAIRS(E, U, J, T)                                                                                    \
   hipExtLaunchKernelGGL((k_pairs<E, false, U, J, T>), dim3(gp), dim3(BLOCK), 0, d->stream, e0, e1, 0, F,           \
-                        d->partials.p, (const double4*)d->Rs4.p, (const int*)d->nbr.p, (const int*)d->nnb.p,       \
+                        d->pairPart, (const double4*)d->Rs4.p, (const int*)d->nbr.p, (const int*)d->nnb.p,       \
                         (const double*)d->charge.p, (const int*)d->chargedFlag.p, pt, cp, c.ntypes, c.L, c.invL2,   \
                         c.Rc2, N, Np, ea, ljt, ljk)
 #define GENERIC_J(E, U, J)                                                                                         \
@@ -2354,16 +2386,20 @@ void dev_compute_pairs(Device* d, const PairCall& c, ForceSums* out) {
   }
   launch_check("pairs");
   // the pair sums have a slot of their own, so that a later post (the
-  // kinetic energy of the kick that follows a deferred call) leaves them
-  d->pairSeq = ++d->seq;
-  hipLaunchKernelGGL(k_reduce_post<4>, dim3(1), dim3(BLOCK), 0, d->stream, d->hpostDev + POST_PAIRS, d->hseqDev,
-                     d->pairSeq, d->partials.p, gp);
+  // kinetic energy of the kick that follows a deferred call) leaves them; in
+  // a deferred call they wait for a small kernel that finishes its own sums
+  // (the kick of the free atoms or the body virial) and takes them along
+  d->pairPending = gp;
+  const bool small = d->bodies.nb > 0 ? d->bodies.nb <= FINISH_BLOCKS * BLOCK
+                                      : N <= (d->uniformFree ? 2 : 1) * FINISH_BLOCKS * BLOCK;
+  if (!c.defer || !small) dev_flush_pairs(d);
   launch_check("reduce");
   if (!c.defer) dev_pairs_result(d, out);
 }
 
 void dev_pairs_result(Device* d, ForceSums* out) {
   if (d->N == 0) { *out = ForceSums{ 0, 0, 0, 0 }; return; }
+  dev_flush_pairs(d);
   post_wait(d, d->pairSeq);
   if (d->profiling) {
     float ms = 0;
@@ -2387,26 +2423,25 @@ void dev_boost(Device* d, int layer, double CP, double CF, bool translate, doubl
   const double* F = d->F.p + 3 * (size_t)Np * layer;
   const int g2 = div_up(div_up(N, 2), BLOCK);
   if (twoKE) {
-    if (d->uniformFree) {
-      hipLaunchKernelGGL(k_boost_u2<true>, dim3(g2), dim3(BLOCK), 0, d->stream, d->P.p, d->partials.p, F, CP, CF,
-                         (int)translate, N, Np, d->invMass0);
-      g = g2;
-    } else {
+    if (d->uniformFree) g = g2;
+    const Post post = dev_post(d, 0, TICKET_KE, g);
+    if (d->uniformFree)
+      hipLaunchKernelGGL(k_boost_u2<true>, dim3(g), dim3(BLOCK), 0, d->stream, d->P.p, d->partials.p, F, CP, CF,
+                         (int)translate, N, Np, d->invMass0, post);
+    else
       hipLaunchKernelGGL(k_boost<true>, dim3(g), dim3(BLOCK), 0, d->stream, d->P.p, d->partials.p, F, d->invMass.p,
-                         d->freeFlag.p, CP, CF, (int)translate, N, Np);
-    }
-    unsigned long long seq = ++d->seq;
-    hipLaunchKernelGGL(k_reduce_post<3>, dim3(1), dim3(BLOCK), 0, d->stream, d->hpostDev, d->hseqDev, seq, d->partials.p, g);
+                         d->freeFlag.p, CP, CF, (int)translate, N, Np, post);
+    dev_post_reduce<3>(d, post, d->partials.p, g);
     launch_check("boost");
-    post_wait(d, seq);
+    post_wait(d, post.seq);
     for (int x = 0; x < 3; x++) twoKE[x] = d->hpost[x];
   } else if (translate) {
     if (d->uniformFree)
       hipLaunchKernelGGL(k_boost_u2<false>, dim3(g2), dim3(BLOCK), 0, d->stream, d->P.p, d->partials.p, F, CP, CF, 1, N,
-                         Np, d->invMass0);
+                         Np, d->invMass0, Post{});
     else
       hipLaunchKernelGGL(k_boost<false>, dim3(g), dim3(BLOCK), 0, d->stream, d->P.p, d->partials.p, F, d->invMass.p,
-                         d->freeFlag.p, CP, CF, 1, N, Np);
+                         d->freeFlag.p, CP, CF, 1, N, Np, Post{});
   }
   launch_check("boost");
 }
@@ -2422,8 +2457,10 @@ void dev_displace(Device* d, double CR, double CP) {
     int g = div_up(div_up(N, 2), BLOCK);
     Scaled sc{ d->trigRs4 ? d->Rs4.p : nullptr, d->trigMixed ? d->Q4.p : nullptr, nullptr, d->type.p, d->charge.p,
                d->chargedFlag.p, d->trigL };
+    const Post post = dev_post(d, POST_TRIG, TICKET_TRIG, g, false);
     hipLaunchKernelGGL(k_displace_u2_trig, dim3(g), dim3(BLOCK), 0, d->stream, d->R.p, d->P.p, CR, CP, N, d->Npad,
-                       d->invMass0, d->R0.p, d->perm.p, d->trigPart.p, sc);
+                       d->invMass0, d->R0.p, d->perm.p, d->trigPart.p, sc, d->trig.p, post);
+    d->trigPreSeq = post.ticket ? post.seq : 0;
     d->trigPreAt = d->posWrites;
     d->trigPreBlocks = g;
     d->trigPreMixed = d->trigMixed;

@@ -119,13 +119,89 @@ __global__ void k_reduce_post(double* __restrict__ host, unsigned long long* __r
   }
 }
 
+// The same totals finished by the producing kernel itself, for grids of at
+// most FINISH_BLOCKS blocks: every block leaves its partial sums and takes a
+// ticket, and the block with the last ticket adds all partials in the order of
+// k_reduce_post (the same totals, bit for bit) and posts them.  The ticket's
+// release and acquire make the partials visible across the XCDs.  The release
+// writes the XCD's L2 back: up to 32 blocks that costs less than the launch it
+// saves (a step of 800 LJ atoms 47 -> 43 us, of 4,000 61 -> 57, of 3,000 water
+// atoms 115 -> 111), at 128 blocks as much, at 200 to 500 more (150,001 LJ
+// atoms 113 -> 125 us, the pair kernel of 1M twice as long), so larger grids
+// keep the second kernel.
+// ticket null: partials only, the caller launches the reduction.
+// The pair sums of an earlier kernel on the stream (pairN blocks of four) ride
+// along and are posted first, which saves their reduction's launch too.
+constexpr int FINISH_BLOCKS = 32;
+struct Post {
+  double* host;
+  unsigned long long* hostSeq;
+  unsigned long long seq;
+  unsigned int* ticket;
+  const double* pairPart;
+  double* pairHost;
+  int pairN;
+};
+// whether this block took the last ticket (all threads call it); the counter
+// is left at zero for the next launch on the stream
+__device__ __forceinline__ bool last_block(unsigned int* ticket, unsigned int nblocks) {
+  __shared__ bool last;
+  if (threadIdx.x == 0) {
+    last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == nblocks - 1;
+    if (last) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  return last;
+}
+// the totals of nb blocks' partials, in the order of k_reduce_post (thread 0)
+template <int NV>
+__device__ __forceinline__ void sum_partials(double (&v)[NV], const double* __restrict__ part, int nb) {
+#pragma unroll
+  for (int k = 0; k < NV; k++) v[k] = 0;
+#pragma unroll 8
+  for (int b = threadIdx.x; b < nb; b += BLOCK) {
+#pragma unroll
+    for (int k = 0; k < NV; k++) v[k] += part[NV * b + k];
+  }
+  block_sum<NV>(v);
+}
+// v: the block's sums in thread 0 (block_sum); called by every thread
+template <int NV>
+__device__ __forceinline__ void finish_sums(const Post& post, double* __restrict__ part, double (&v)[NV], int blk) {
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int k = 0; k < NV; k++) part[NV * blk + k] = v[k];
+  }
+  if (!post.ticket || !last_block(post.ticket, gridDim.x)) return;
+  if (post.pairN) {
+    double w[4] = { 0, 0, 0, 0 };
+    sum_partials<4>(w, post.pairPart, post.pairN);
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) post.pairHost[k] = w[k];
+    }
+    __syncthreads();
+  }
+  sum_partials<NV>(v, part, gridDim.x);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int k = 0; k < NV; k++) post.host[k] = v[k];
+    __threadfence_system();
+    *(volatile unsigned long long*)post.hostSeq = post.seq;
+  }
+}
+
 // ------------------------------------------------------------ device state
 
 // Slots in the posted-results block (64 doubles): the pair sums, the Ewald
 // energy and virial, the learned model's energy, virial and overflow flag,
 // the rigid bodies' kinetic-energy terms and their virial, the model's
-// low-k energy and virial; the other posts use slot 0.
-constexpr int POST_PAIRS = 8, POST_EWALD = 16, POST_MODEL = 24, POST_BODY_KE = 32, POST_BODY_W = 40, POST_LOWK = 48;
+// low-k energy and virial, the rebuild trigger; the kick's kinetic energy uses
+// slot 0.
+constexpr int POST_PAIRS = 8, POST_EWALD = 16, POST_MODEL = 24, POST_BODY_KE = 32, POST_BODY_W = 40, POST_LOWK = 48,
+              POST_TRIG = 56;
+// Tickets of the kernels that finish their own sums
+enum { TICKET_KE, TICKET_TRIG, TICKET_BODY_KE, TICKET_BODY_W, TICKETS };
 
 template <typename T>
 struct DBuf {
@@ -203,6 +279,9 @@ struct Device {
   unsigned long long* hseqDev = nullptr;
   unsigned long long seq = 0;
   unsigned long long pairSeq = 0;   // post of the last pair evaluation (slot POST_PAIRS)
+  int pairPending = 0;              // blocks of a pair evaluation whose sums are not reduced yet (0: none)
+  double* pairPart = nullptr;       // the pair kernels' partial sums (after the other partials)
+  size_t pairPartSize = 0;
   // per layer: FP32 records {c0, c1, c2, eshift} and Coulomb factors of the
   // type pairs, used by the mixed kernels when ljcOk (k_pairs_mx, LJ = 2)
   DBuf<float4> ljt;
@@ -210,7 +289,9 @@ struct Device {
   DBuf<double4> ljt64;   // the same records in FP64 for the FP64 kernels
   DBuf<double> ljk64;
   std::vector<char> ljcOk;
-  unsigned long long trigSeq = 0;   // post of the last rebuild trigger (slot 0)
+  unsigned long long trigSeq = 0;   // post of the last rebuild trigger (slot POST_TRIG)
+  unsigned long long trigPreSeq = 0;   // ... posted by the drift itself (0: pass A only)
+  unsigned int* tickets = nullptr;  // one counter per TICKET_*, zero between launches (after trig)
   // Every write of R on the device counts in posWrites.  The drift of
   // uniform free atoms forms the next trigger's pass A (partials, scaled
   // positions) on the way, with the set-up of the last trigger (trigMixed,
@@ -244,6 +325,37 @@ struct Device {
 
 
 void launch_check(const char* what);
+// Where a kernel of `blocks` blocks posts its totals, under the next sequence
+// number; no ticket when the grid is too large to finish them itself.  Pair
+// sums that wait for their reduction go along (sums: the kernel ends in
+// finish_sums).
+inline Post dev_post(Device* d, int slot, int ticket, int blocks, bool sums = true) {
+  Post p{ d->hpostDev + slot, d->hseqDev, ++d->seq, nullptr, nullptr, nullptr, 0 };
+  if (blocks > FINISH_BLOCKS) return p;
+  p.ticket = d->tickets + ticket;
+  if (sums && d->pairPending) {
+    p.pairPart = d->pairPart;
+    p.pairHost = d->hpostDev + POST_PAIRS;
+    p.pairN = d->pairPending;
+    d->pairPending = 0;
+    d->pairSeq = p.seq;
+  }
+  return p;
+}
+// ... whose reduction is launched here when the kernel does not finish it
+template <int NV>
+inline void dev_post_reduce(Device* d, const Post& post, const double* part, int blocks) {
+  if (!post.ticket)
+    hipLaunchKernelGGL(k_reduce_post<NV>, dim3(1), dim3(BLOCK), 0, d->stream, post.host, post.hostSeq, post.seq, part, blocks);
+}
+// Pair sums that no later kernel took along are reduced and posted now.
+inline void dev_flush_pairs(Device* d) {
+  if (!d->pairPending) return;
+  d->pairSeq = ++d->seq;
+  hipLaunchKernelGGL(k_reduce_post<4>, dim3(1), dim3(BLOCK), 0, d->stream, d->hpostDev + POST_PAIRS, d->hseqDev,
+                     d->pairSeq, d->pairPart, d->pairPending);
+  d->pairPending = 0;
+}
 // Waits until the post with sequence number seq has arrived in pinned host
 // memory (posts arrive in stream order).
 void dev_post_wait(Device* d, unsigned long long seq);

@@ -638,7 +638,7 @@ __global__ void k_body_update(BodyState B, double* __restrict__ R, const int* __
 // with the body parts of kinetic_energies (EmDeeData.f90:900-922).
 template <bool KE>
 __global__ void k_body_boost(BodyState B, const double* __restrict__ F, const int* __restrict__ iperm, double CP,
-                             double CF, int translate, int rotate, int Npad) {
+                             double CF, int translate, int rotate, int Npad, Post post) {
   int b = blockIdx.x * blockDim.x + threadIdx.x;
   double v[6] = { 0, 0, 0, 0, 0, 0 };
   if (b < B.nb) {
@@ -676,7 +676,7 @@ __global__ void k_body_boost(BodyState B, const double* __restrict__ F, const in
   }
   if (KE) {
     block_sum<6>(v);
-    if (threadIdx.x == 0) for (int k = 0; k < 6; k++) B.part.p[6 * blockIdx.x + k] = v[k];
+    finish_sums<6>(post, B.part.p, v, blockIdx.x);
   }
 }
 
@@ -709,7 +709,8 @@ __global__ void __launch_bounds__(BLOCK) k_body_move(BodyState B, double* __rest
 }
 
 // rigid_body_virial partials: EmDeeData.f90:926-953
-__global__ void k_body_virial(BodyState B, const double* __restrict__ F, const int* __restrict__ iperm, int Npad) {
+__global__ void k_body_virial(BodyState B, const double* __restrict__ F, const int* __restrict__ iperm, int Npad,
+                              Post post) {
   int b = blockIdx.x * blockDim.x + threadIdx.x;
   double v[1] = { 0 };
   if (b < B.nb) {
@@ -720,7 +721,7 @@ __global__ void k_body_virial(BodyState B, const double* __restrict__ F, const i
     }
   }
   block_sum<1>(v);
-  if (threadIdx.x == 0) B.part.p[blockIdx.x] = v[0];
+  finish_sums<1>(post, B.part.p, v, blockIdx.x);
 }
 
 // assign_momenta for bodies from particle momenta (EmDeeData.f90:157-189);
@@ -918,15 +919,16 @@ void dev_bodies_boost(Device* d, int layer, double CP, double CF, bool translate
   int g = div_up(B.nb, BLOCK);
   const double* F = d->F.p + 3 * (size_t)d->Npad * layer;
   if (twoKE6) {
-    hipLaunchKernelGGL(k_body_boost<true>, dim3(g), dim3(BLOCK), 0, d->stream, B, F, d->iperm.p, CP, CF, (int)translate, (int)rotate, d->Npad);
-    // the totals straight into pinned host memory (same fixed-order sums)
-    const unsigned long long seq = ++d->seq;
-    hipLaunchKernelGGL(k_reduce_post<6>, dim3(1), dim3(BLOCK), 0, d->stream, d->hpostDev + POST_BODY_KE, d->hseqDev, seq,
-                       B.part.p, g);
-    dev_post_wait(d, seq);
+    // the totals straight into pinned host memory
+    const Post post = dev_post(d, POST_BODY_KE, TICKET_BODY_KE, g);
+    hipLaunchKernelGGL(k_body_boost<true>, dim3(g), dim3(BLOCK), 0, d->stream, B, F, d->iperm.p, CP, CF, (int)translate,
+                       (int)rotate, d->Npad, post);
+    dev_post_reduce<6>(d, post, B.part.p, g);
+    dev_post_wait(d, post.seq);
     for (int k = 0; k < 6; k++) twoKE6[k] = d->hpost[POST_BODY_KE + k];
   } else {
-    hipLaunchKernelGGL(k_body_boost<false>, dim3(g), dim3(BLOCK), 0, d->stream, B, F, d->iperm.p, CP, CF, (int)translate, (int)rotate, d->Npad);
+    hipLaunchKernelGGL(k_body_boost<false>, dim3(g), dim3(BLOCK), 0, d->stream, B, F, d->iperm.p, CP, CF, (int)translate, (int)rotate, d->Npad,
+                       Post{});
   }
   launch_check("body boost");
 }
@@ -944,10 +946,10 @@ void dev_bodies_virial_launch(Device* d, int layer) {
   BodyState& B = d->bodies;
   if (B.nb == 0) { d->hpost[POST_BODY_W] = 0.0; return; }
   int g = div_up(B.nb, BLOCK);
-  hipLaunchKernelGGL(k_body_virial, dim3(g), dim3(BLOCK), 0, d->stream, B, d->F.p + 3 * (size_t)d->Npad * layer, d->iperm.p, d->Npad);
-  const unsigned long long seq = ++d->seq;
-  hipLaunchKernelGGL(k_reduce_post<1>, dim3(1), dim3(BLOCK), 0, d->stream, d->hpostDev + POST_BODY_W, d->hseqDev, seq,
-                     B.part.p, g);
+  const Post post = dev_post(d, POST_BODY_W, TICKET_BODY_W, g);
+  hipLaunchKernelGGL(k_body_virial, dim3(g), dim3(BLOCK), 0, d->stream, B, d->F.p + 3 * (size_t)d->Npad * layer, d->iperm.p,
+                     d->Npad, post);
+  dev_post_reduce<1>(d, post, B.part.p, g);
 }
 
 double dev_bodies_virial_read(const Device* d) { return -d->hpost[POST_BODY_W]; }
