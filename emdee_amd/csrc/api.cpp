@@ -368,8 +368,9 @@ static bool forces_begin(tEmDee* md, bool defer, ForceSums& fs) {
   }
   bool rebuild = dev_trigger_result(me->dev, me->skinSq);
   if (rebuild) {
-    dev_rebuild(me->dev, me->L, me->xRc, std::sqrt(me->xInRcSq));
+    dev_rebuild(me->dev, me->L, me->xRc, me->Rc, me->precision != 0);
     md->Builds += 1;
+    c.fresh = 1;
   }
   md->Time.Neighbor += wtime();
   md->Time.Pair -= wtime();

@@ -501,11 +501,11 @@ template <bool SIMPLE>
 __device__ __forceinline__ bool list_accept(int j, int4 qj, int bj, int i, int4 qi, int ti, int bi,
                                             const double4* __restrict__ Rs4, const int* __restrict__ perm,
                                             const uint8_t* __restrict__ interact, const int* __restrict__ exItem,
-                                            int e0, int e1, int ntypes, double xRc2, float lo, float hi) {
+                                            int e0, int e1, int ntypes, double xRc2, float lo, float hi, float& r2) {
   float dx = (float)(int)((unsigned int)qi.x - (unsigned int)qj.x);
   float dy = (float)(int)((unsigned int)qi.y - (unsigned int)qj.y);
   float dz = (float)(int)((unsigned int)qi.z - (unsigned int)qj.z);
-  float r2 = dx * dx + dy * dy + dz * dz;
+  r2 = dx * dx + dy * dy + dz * dz;
   bool odd = ((qi.w | qj.w) & Q4_NONFINITE) != 0;
   bool in = r2 < lo && !odd;
   if (!in && (r2 < hi || odd)) in = exact_inside(Rs4, i, j, xRc2);
@@ -528,8 +528,9 @@ __device__ __forceinline__ void scan_range(int a, int b, int i, double xi, doubl
                                            const int4* __restrict__ Q4, int4 qi, float lo, float hi) {
   if (S > 1) {
     auto accept = [&](int j) -> bool {
+      float r2;
       return list_accept<SIMPLE>(j, Q4[j], SIMPLE ? 0 : body[j], i, qi, ti, bi, Rs4, perm, interact, exItem, e0, e1,
-                                 ntypes, xRc2, lo, hi);
+                                 ntypes, xRc2, lo, hi, r2);
     };
     const int lane = threadIdx.x & 63, sub = lane & (S - 1), gbase = lane & ~(S - 1);
     for (int j0 = a; j0 < b; j0 += S) {
@@ -607,14 +608,56 @@ __device__ __forceinline__ void scan_range(int a, int b, int i, double xi, doubl
   }
   for (; j < b; j++) test(j, Rs4[j]);
 }
-template <bool SIMPLE, int S>
+// Shells.  The 16-lane build orders an atom's list by the distance at the
+// build: r < rc + skin/4, then three shells of skin/4 each (nsh: running
+// counts).  Two atoms have approached by at most twice the largest
+// displacement since the build, which the trigger finds at every force
+// evaluation, so the pair kernels stop at the first shell that cannot hold a
+// pair inside the cutoff yet (list_count); the pair set is the same.  Water's
+// lists (rc 10 A, skin 2 A) hold 726 entries, 420 of them inside rc: the
+// kernels read 486, 560, 640 or 726 of them as the displacement grows, and
+// entries inside the cutoff lie together, so fewer waves run the pair terms
+// for a few lanes only.  12,288 atoms: pair kernel 60 -> 49 us, build 60 -> 69
+// us every ten steps.
+// The near entries go straight to the list in scan order, the others to LDS
+// until the atom's scan ends and are then sorted by shell; past FAR_CAP they
+// go to the near part, which is always read.  (98,304 atoms: FAR_CAP 160
+// leaves LDS for six blocks per CU instead of five: build 302 us for 353, pair
+// kernel 341 for 314; the entries kept in global memory instead: build 398 us;
+// a scan over the lanes that places all four parts at once: 444 us.)
+// Where the order changes, so does the rounding of the sums.  Lists for the
+// mixed form keep the scan order: its FP32 sums of four entries follow the
+// list.  So do systems of more than SHELL_ATOMS atoms, though 98,304 would gain
+// (pair kernel 398 -> 314 us, build 269 -> 353 us): among so many molecules a
+// few amplify a rounding so fast that momenta moved by 4e-8 within 20 steps of
+// 2 fs, where every other change of order stays below 1e-9.
+constexpr int FAR_CAP = 300;   // 32 KB of LDS a block: five blocks per CU
+constexpr int SHELL_ATOMS = 16384;
+struct ShellCut {            // for the pair kernels
+  const int4* nsh;           // null: lists without shells
+  const double* trig;        // [0]: largest squared displacement since the build
+  double rc, e1, e2, e3;     // cutoff of the layer; inner edges of the shells
+  int fresh;                 // the list has just been built: no displacement
+};
+__device__ __forceinline__ int list_count(const ShellCut& sc, const int* __restrict__ nnb, int i) {
+  if (!sc.nsh) return nnb[i];
+  const int4 c = sc.nsh[i];
+  const double reach = sc.rc + (sc.fresh ? 0.0 : 2.0 * sqrt(sc.trig[0]));
+  return reach < sc.e1 ? c.x : reach < sc.e2 ? c.y : reach < sc.e3 ? c.z : c.w;
+}
+// x of the lane `ctrl` away in the row of 16 lanes, 0 outside the row
+template <int CTRL>
+__device__ __forceinline__ unsigned row_dpp(unsigned x) {
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, true);
+}
+template <bool SIMPLE, int S, bool SHELL>
 __global__ void __launch_bounds__(BLOCK)
 k_build_list(int* __restrict__ nbr, int* __restrict__ nnb, int* __restrict__ flags, double* __restrict__ part,
              const double4* __restrict__ Rs4, const int* __restrict__ key, const int* __restrict__ start,
              const int* __restrict__ body, const int* __restrict__ perm,
              const uint8_t* __restrict__ interact, const int* __restrict__ exOff, const int* __restrict__ exItem,
              int nexcl, int ntypes, int M, double xRc2, int cap, int N, int Npad, const int4* __restrict__ Q4,
-             float lo, float hi) {
+             float lo, float hi, int4* __restrict__ nsh, float3 edge) {
   int blk = xcd_block();
   int gt = blk * BLOCK + threadIdx.x;
   int i = S == 1 ? gt : gt / S, sub = S == 1 ? 0 : gt % S;
@@ -725,20 +768,71 @@ k_build_list(int* __restrict__ nbr, int* __restrict__ nnb, int* __restrict__ fla
       int j = has ? ca + off : i;
       int4 qj = q4At(j);
       int bj = SIMPLE ? 0 : bodyAt(j);
-      for (int step = 0; step < steps; step++) {
-        off += S;
-        settle();
-        const bool hasN = s < nseg;
-        const int jN = hasN ? ca + off : i;
-        const int4 qN = q4At(jN);
-        const int bN = SIMPLE ? 0 : bodyAt(jN);
-        bool ok = has && list_accept<SIMPLE>(j, qj, bj, i, qi, ti, bi, Rs4, perm, interact, exItem, e0, e1, ntypes,
-                                             xRc2, lo, hi);
-        unsigned g = (unsigned)(__ballot(ok) >> gbase) & gmask;
-        int pos = cnt + __popc(g & lower);
-        if (ok && pos < cap) nbr[nb_at(pos, i, Npad)] = j;
-        cnt += __popc(g);
-        has = hasN; j = jN; qj = qN; bj = bN;
+      if constexpr (!SHELL) {
+        for (int step = 0; step < steps; step++) {
+          off += S;
+          settle();
+          const bool hasN = s < nseg;
+          const int jN = hasN ? ca + off : i;
+          const int4 qN = q4At(jN);
+          const int bN = SIMPLE ? 0 : bodyAt(jN);
+          float r2;
+          bool ok = has && list_accept<SIMPLE>(j, qj, bj, i, qi, ti, bi, Rs4, perm, interact, exItem, e0, e1, ntypes,
+                                               xRc2, lo, hi, r2);
+          unsigned g = (unsigned)(__ballot(ok) >> gbase) & gmask;
+          int pos = cnt + __popc(g & lower);
+          if (ok && pos < cap) nbr[nb_at(pos, i, Npad)] = j;
+          cnt += __popc(g);
+          has = hasN; j = jN; qj = qN; bj = bN;
+        }
+      } else {
+        // n0 entries of the near part are in the list, nf of the shells in LDS
+        // with their shell in the top bits (both uniform over the atom's lanes)
+        __shared__ unsigned farBuf[BLOCK / S][FAR_CAP];
+        unsigned* fb = farBuf[threadIdx.x / S];
+        int n0 = 0, nf = 0;
+        for (int step = 0; step < steps; step++) {
+          off += S;
+          settle();
+          const bool hasN = s < nseg;
+          const int jN = hasN ? ca + off : i;
+          const int4 qN = q4At(jN);
+          const int bN = SIMPLE ? 0 : bodyAt(jN);
+          float r2 = 0.0f;
+          const bool ok = has && list_accept<SIMPLE>(j, qj, bj, i, qi, ti, bi, Rs4, perm, interact, exItem, e0, e1, ntypes,
+                                                     xRc2, lo, hi, r2);
+          const bool out = ok && r2 >= edge.x && nf <= FAR_CAP - S, in = ok && !out;
+          const unsigned g = (unsigned)(__ballot(in) >> gbase) & gmask, gf = (unsigned)(__ballot(out) >> gbase) & gmask;
+          const int pos = n0 + __popc(g & lower);
+          if (in && pos < cap) nbr[nb_at(pos, i, Npad)] = j;
+          if (out) fb[nf + __popc(gf & lower)] = (unsigned)j | (r2 < edge.y ? 0u : r2 < edge.z ? 1u << 30 : 2u << 30);
+          n0 += __popc(g);
+          nf += __popc(gf);
+          has = hasN; j = jN; qj = qN; bj = bN;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        // the shells behind the near part: each lane counts its entries per
+        // shell (ten bits each), a scan over the lanes gives their places
+        unsigned mine = 0;
+        for (int e = sub; e < nf; e += S) mine += 1u << (10 * (fb[e] >> 30));
+        unsigned sum = mine;
+        sum += row_dpp<0x111>(sum);   // row_shr 1, 2, 4, 8: inclusive scan
+        sum += row_dpp<0x112>(sum);
+        sum += row_dpp<0x114>(sum);
+        sum += row_dpp<0x118>(sum);
+        const unsigned all = row_dpp<0x15F>(sum), before = sum - mine;   // row_newbcast 15
+        const int m1 = n0 + (int)(all & 1023u), m2 = m1 + (int)((all >> 10) & 1023u);
+        cnt = n0 + nf;
+        int p0 = n0 + (int)(before & 1023u), p1 = m1 + (int)((before >> 10) & 1023u), p2 = m2 + (int)(before >> 20);
+        for (int e = sub; e < nf; e += S) {
+          const unsigned v = fb[e], k = v >> 30;
+          const int pos = k == 0 ? p0 : k == 1 ? p1 : p2;
+          p0 += k == 0; p1 += k == 1; p2 += k == 2;
+          if (pos < cap) nbr[nb_at(pos, i, Npad)] = (int)(v & 0x3fffffffu);
+        }
+        if (sub == 0) nsh[i] = make_int4(n0, m1, m2, cnt);
       }
     } else {
       // the cell starts of the next row are loaded before the current row is
@@ -1147,7 +1241,7 @@ k_pairs(double* __restrict__ F, double* __restrict__ partials,
         const double* __restrict__ charge, const int* __restrict__ charged,
         const DevPair* __restrict__ pairs, const DevCoul* __restrict__ coulp,
         int ntypes, double L, double invL2, double Rc2, int N, int Npad, double* __restrict__ eatom,
-        const double4* __restrict__ ljt, const double* __restrict__ ljk) {
+        const double4* __restrict__ ljt, const double* __restrict__ ljk, ShellCut sc) {
   using T = typename std::conditional<MIXED, float, double>::type;
   int blk = xcd_block();
   int gt = blk * BLOCK + threadIdx.x;
@@ -1176,7 +1270,7 @@ k_pairs(double* __restrict__ F, double* __restrict__ partials,
     const DevPair* srow = spair + ti * ntypes;
     DevPair pu;
     if (UNIFORM) pu = pairs[0];   // uniform address: scalar loads
-    const int n = nnb[i];
+    const int n = TPA == 1 ? nnb[i] : list_count(sc, nnb, i);
     // qjp: the neighbour's charge when the caller loaded it with the position
     // (LJ == 2 on the multi-lane path), else read here
     auto one = [&](int j, const double4& rj, double qjp = 0.0, bool haveQ = false) {
@@ -1333,7 +1427,7 @@ k_pairs_mx(double* __restrict__ F, double* __restrict__ partials, const int4* __
            const int* __restrict__ nnb, const float* __restrict__ qf, const DevPair* __restrict__ pairs,
            const DevCoul* __restrict__ coulp,
            int ntypes, MixedCut mc, int N, int Npad, double* __restrict__ eatom, const float4* __restrict__ ljt,
-           const float* __restrict__ ljk) {
+           const float* __restrict__ ljk, ShellCut sc) {
   int blk = xcd_block();
   int gt = blk * BLOCK + threadIdx.x;
   int i = TPA == 1 ? gt : gt / TPA, sub = TPA == 1 ? 0 : gt % TPA;
@@ -1346,7 +1440,7 @@ k_pairs_mx(double* __restrict__ F, double* __restrict__ partials, const int4* __
     const int trow = (qi.w & Q4_TYPE) * ntypes;
     DevPair pu;
     if (UNIFORM) pu = pairs[0];   // uniform address: scalar loads, no VGPRs
-    const int n = nnb[i];
+    const int n = TPA == 1 ? nnb[i] : list_count(sc, nnb, i);
     auto one = [&](int j, const int4& qj, MixedAcc& a) {
       float dx = (float)(int)((unsigned int)qi.x - (unsigned int)qj.x);
       float dy = (float)(int)((unsigned int)qi.y - (unsigned int)qj.y);
@@ -1900,7 +1994,7 @@ void dev_destroy(Device* d) {
   if (!d) return;
   (void)hipStreamSynchronize(d->stream);
   for (DBuf<double>* b : { &d->R, &d->P, &d->R0, &d->invMass, &d->charge, &d->F, &d->tmp3, &d->tmpF, &d->tmp1, &d->tmpP, &d->tmpQ, &d->stage, &d->partials, &d->trigPart, &d->result, &d->trig, &d->shadow }) b->release();
-  d->Rs4.release(); d->Q4.release(); d->P16.release(); d->qf.release(); d->eatom.release();
+  d->nsh.release(); d->Rs4.release(); d->Q4.release(); d->P16.release(); d->qf.release(); d->eatom.release();
   for (DBuf<int>* b : { &d->type, &d->body, &d->perm, &d->freeFlag, &d->chargedFlag, &d->tmpI, &d->tmpBody, &d->tmpPerm, &d->tmpFree, &d->tmpCharged, &d->key, &d->cellCount, &d->cellStart, &d->order, &d->blockSums, &d->nbr, &d->nnb, &d->flags, &d->exOff, &d->exItem, &d->iperm }) b->release();
   d->pairs.release(); d->couls.release(); d->interact.release(); d->ljt.release(); d->ljk.release(); d->ljt64.release();
   d->ljk64.release();
@@ -2133,8 +2227,7 @@ static void ensure_cells(Device* d, int M) {
   d->blockSums.alloc(div_up(d->ncells + 1, BLOCK) + 1);
 }
 
-void dev_rebuild(Device* d, double L, double xRc, double xInRc) {
-  (void)xInRc;
+void dev_rebuild(Device* d, double L, double xRc, double rc, bool mixed) {
   int N = d->N, Np = d->Npad;
   if (N == 0) return;
   d->posWrites++;                      // R and R0 in a new slot order
@@ -2202,6 +2295,16 @@ void dev_rebuild(Device* d, double L, double xRc, double xInRc) {
   double xRc2 = (xRc * xRc) / (L * L);
   const double two32 = 4294967296.0, rc2u = xRc2 * two32 * two32, band = band_rel(xRc2);
   float lo = (float)(rc2u * (1.0 - band)), hi = (float)(rc2u * (1.0 + band));
+  // inner edges of the three outer shells
+  float3 edge;
+  for (int k = 0; k < 3; k++) {
+    const double e = rc + 0.25 * (k + 1) * (xRc - rc);
+    d->shellEdge[k] = e * (1.0 - 1e-5);
+    (&edge.x)[k] = (float)(e * e / (L * L) * two32 * two32);
+  }
+  d->shells = S == 16 && !mixed && N <= SHELL_ATOMS;
+  d->listL = L;
+  if (d->shells) d->nsh.alloc(Np);
   if (d->cap == 0) {
     d->cap = std::max(32, (int)(1.35 * vol + 16));
     d->cap = (d->cap + 7) & ~7;
@@ -2220,14 +2323,17 @@ void dev_rebuild(Device* d, double L, double xRc, double xInRc) {
                             d->flags.p, d->partials.p, (const double4*)d->Rs4.p, (const int*)d->key.p,
                             (const int*)d->cellStart.p, M, xRc2, d->cap, N, Np, (const uint2*)d->P16.p, lo16, hi16);
     } else {
-      auto kern = simple ? (S == 16 ? k_build_list<true, 16> : S == 4 ? k_build_list<true, 4> : k_build_list<true, 1>)
-                         : (S == 16 ? k_build_list<false, 16> : S == 4 ? k_build_list<false, 4> : k_build_list<false, 1>);
+      auto kern = d->shells ? (simple ? k_build_list<true, 16, true> : k_build_list<false, 16, true>)
+                  : simple  ? (S == 16 ? k_build_list<true, 16, false>
+                                       : S == 4 ? k_build_list<true, 4, false> : k_build_list<true, 1, false>)
+                            : (S == 16 ? k_build_list<false, 16, false>
+                                       : S == 4 ? k_build_list<false, 4, false> : k_build_list<false, 1, false>);
       hipExtLaunchKernelGGL(kern, dim3(gl), dim3(BLOCK), 0, d->stream, e0, e1, 0, d->nbr.p, d->nnb.p, d->flags.p,
                             d->partials.p, (const double4*)d->Rs4.p, (const int*)d->key.p, (const int*)d->cellStart.p,
                             (const int*)d->body.p, (const int*)d->perm.p,
                             d->allInteract ? nullptr : (const uint8_t*)d->interact.p,
                             (const int*)d->exOff.p, (const int*)d->exItem.p, d->nexcl, d->ntypes, M, xRc2, d->cap, N, Np,
-                            (const int4*)d->Q4.p, lo, hi);
+                            (const int4*)d->Q4.p, lo, hi, d->nsh.p, edge);
     }
     launch_check("build_list");
     hipLaunchKernelGGL(k_reduce_partials<1>, dim3(1), dim3(BLOCK), 0, d->stream, d->result.p + 8, d->partials.p, gl);
@@ -2314,6 +2420,11 @@ void dev_compute_pairs(Device* d, const PairCall& c, ForceSums* out) {
   if ((size_t)gp * 4 > d->pairPartSize) fatal("compute_forces", "too many lanes per atom for the partial sums");
   double* ea = d->wantAtomE ? d->eatom.p : nullptr;
   int variant = (c.energy ? 4 : 0) + (U ? 2 : 0) + (LJ ? 1 : 0);
+  // inner edges of the shells a part in 10^5 low, far above the rounding of
+  // the build's FP32 distances; no shells once the box has changed (a pair's
+  // image then moves with it)
+  ShellCut sc{ d->shells && d->listL == c.L ? d->nsh.p : nullptr, d->trig.p, std::sqrt(c.Rc2) * c.L,
+               d->shellEdge[0], d->shellEdge[1], d->shellEdge[2], c.fresh };
   if (c.mixed) {
     // cutoff in fixed-point units: Rc2 (scaled) * 2^64
     MixedCut mc;
@@ -2331,7 +2442,7 @@ void dev_compute_pairs(Device* d, const PairCall& c, ForceSums* out) {
   hipExtLaunchKernelGGL((k_pairs_mx<E, U, J, T>), dim3(gp), dim3(BLOCK), 0, d->stream, e0, e1, 0, F,                \
                         d->pairPart, (const int4*)d->Q4.p, (const double*)d->R.p, (const double4*)d->Rs4.p,     \
                         (const int*)d->nbr.p, (const int*)d->nnb.p, (const float*)d->qf.p, pt, cp, c.ntypes, mc, N, \
-                        Np, ea, ljt, ljk)
+                        Np, ea, ljt, ljk, sc)
 #define GENERIC_MX_J(E, U, J)                                                                                      \
   do {                                                                                                            \
     if (tpa == 64) LAUNCH_MX(E, U, J, 64); else if (tpa == 32) LAUNCH_MX(E, U, J, 32);                            \
@@ -2361,7 +2472,7 @@ void dev_compute_pairs(Device* d, const PairCall& c, ForceSums* out) {
   hipExtLaunchKernelGGL((k_pairs<E, false, U, J, T>), dim3(gp), dim3(BLOCK), 0, d->stream, e0, e1, 0, F,           \
                         d->pairPart, (const double4*)d->Rs4.p, (const int*)d->nbr.p, (const int*)d->nnb.p,       \
                         (const double*)d->charge.p, (const int*)d->chargedFlag.p, pt, cp, c.ntypes, c.L, c.invL2,   \
-                        c.Rc2, N, Np, ea, ljt, ljk)
+                        c.Rc2, N, Np, ea, ljt, ljk, sc)
 #define GENERIC_J(E, U, J)                                                                                         \
   do {                                                                                                            \
     if (tpa == 64) LAUNCH_PAIRS(E, U, J, 64); else if (tpa == 32) LAUNCH_PAIRS(E, U, J, 32);                      \

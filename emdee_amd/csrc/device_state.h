@@ -252,6 +252,9 @@ struct Device {
   // neighbor list
   int cap = 0;
   DBuf<int> nbr, nnb;
+  DBuf<int4> nsh;         // running counts of an atom's near part and shells (k_build_list)
+  bool shells = false;    // the current list has them
+  double shellEdge[3] = { 0, 0, 0 }, listL = 0;
   DBuf<int> flags;        // [0] overflow max count
   bool built = false;
   long listVersion = 0;   // incremented at every list build

@@ -82,6 +82,7 @@ struct PairCall {
   int mixed;          // FP32 pair arithmetic with FP64 accumulation
   double L, invL2, Rc2;   // box and scaled squared cutoff
   int scaled;         // scaled positions are current (written by the trigger or the list build)
+  int fresh = 0;      // the list was built for these positions
   int defer = 0;      // return once the kernels are queued; dev_pairs_result reads the sums
 };
 
@@ -123,7 +124,7 @@ void dev_trigger_launch(Device* d, double L, bool mixed, int layer);
 bool dev_trigger_result(Device* d, double skinSq);
 // Whether the last steps' trigger values make a rebuild at this step unlikely.
 bool dev_trigger_unlikely(const Device* d, double skinSq);
-void dev_rebuild(Device* d, double L, double xRc, double xInRc);  // sort + full Verlet list
+void dev_rebuild(Device* d, double L, double xRc, double rc, bool mixed);  // sort + full Verlet list
 int dev_neighbor_pairs(Device* d, int max, int* out);             // half set, 1-based i<j
 
 // Forces of one layer: fills F(layer) and returns the reduced sums.
