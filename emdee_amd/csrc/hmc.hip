@@ -59,6 +59,12 @@ struct ReplicaDesc {
   double Rc2s, unit;       // FP64 scaled cutoff; L / 2^32
   double Rl2s, trig2s;     // list radius (rc + skin)^2 and (skin/2)^2, scaled units^2
 };
+// per-atom vectors of all replicas, component by component: x of atom i at
+// [i], y at [total + i], z at [2 total + i]
+struct HmcState {
+  double *R, *P, *F, *Rsave, *Fsave;
+  size_t total;
+};
 constexpr double HMC_SKIN = 0.3;   // list skin (LJ units; 0.2 and 0.45 measured slower)
 
 __host__ __device__ inline uint64_t mix64(uint64_t z) {
@@ -94,58 +100,81 @@ __device__ double block_total(double v, double* red) {
 }
 }  // namespace
 
+// LDS of a workgroup.  qz lies below qxy so that both are reached from a list
+// entry (8 j, the byte offset of qxy[j]) with constant offsets.
+struct HmcLds {
+  unsigned int qz[HMC_NMAX];
+  uint2 qxy[HMC_NMAX];
+  unsigned short clist[HMC_NMAX];
+  unsigned short cstart[HMC_CMAX + 2];
+  unsigned int ccount2[HMC_CMAX / 2];   // 16-bit cell counts, two per word
+};
+
 // One HMC workgroup per replica.  mode 0: forces and potential energy of the
 // current coordinates only; mode 1: ncycles full cycles.
+//
+// A step is two passes over the atoms with a barrier after each.  The force
+// pass walks an atom's list and gives it both half kicks that its force takes
+// part in (the end of this step and the start of the next), so forces stay in
+// registers except at a trajectory's end; the drift pass moves the atom and
+// renews its fixed-point coordinates.  Per step and atom that is 120 bytes of
+// state instead of 370.  The list holds packets of eight 16-bit entries, one
+// 16-byte load each (four, and the next in flight, instead of eight loads with
+// an address and a bound test apiece), padded with the atom itself, which the
+// pair terms mask.  Bound by instruction issue and the latency of one
+// replica's 16 wavefronts per CU: half the time is the force pass, 45 % the
+// 1.7 list builds of a cycle.  512 replicas of 256 to 8,192 atoms, ten steps:
+// 4.41 -> 3.82 ms a cycle.  Partners read two, four or eight at a time and
+// masked instead of branched over: 3.93, 4.11 and 4.04 ms with 1,024 threads,
+// 10 % less with 256, which no replica set of these sizes chooses.
 template <int BS, int DIV, bool MIXED>
 __global__ void __launch_bounds__(BS)
-k_hmc(const ReplicaDesc* __restrict__ desc, const int* __restrict__ order, double4* __restrict__ R,
-      double4* __restrict__ P, double4* __restrict__ F, double4* __restrict__ Rsave, double4* __restrict__ Fsave,
-      double* __restrict__ U, int* __restrict__ cycle, long long* __restrict__ accepted,
-      double* __restrict__ lastDH, double rc, double dt, int nsteps, uint64_t seed, int ncycles, int mode,
-      unsigned short* __restrict__ nlist, unsigned short* __restrict__ nnb, uint4* __restrict__ qbuild, int cap,
-      int* __restrict__ lstate, double* __restrict__ Uhist, int histLen) {
-  __shared__ unsigned int qx[HMC_NMAX], qy[HMC_NMAX], qz[HMC_NMAX];
-  __shared__ unsigned short clist[HMC_NMAX];
-  __shared__ int cstart[HMC_CMAX + 1];
-  __shared__ unsigned int ccount2[HMC_CMAX / 2];   // 16-bit cell counts, two per word
+k_hmc(const ReplicaDesc* __restrict__ desc, const int* __restrict__ order, HmcState st, double* __restrict__ U,
+      int* __restrict__ cycle, long long* __restrict__ accepted, double* __restrict__ lastDH, double dt, int nsteps,
+      uint64_t seed, int ncycles, int mode, unsigned short* __restrict__ nlist, unsigned short* __restrict__ nnb,
+      uint4* __restrict__ qbuild, int cap, int* __restrict__ lstate, double* __restrict__ Uhist, int histLen) {
+  __shared__ HmcLds s;
   __shared__ double red[BS / 64];
-  __shared__ int scanTmp[BS];
+  __shared__ int scanTmp[BS / 64];
   __shared__ int cycleNow;
   __shared__ double Unow;
-  __shared__ int listState;   // 0: no valid list, 1: valid list, 2: overflow (cell walk)
+  __shared__ int listState;   // 0: no valid list, 1: valid list, 2: overflow (every atom)
 
   const int r = order[blockIdx.x];
   const ReplicaDesc d = desc[r];
   const int N = d.N;
-  double4* Rr = R + d.off;
-  double4* Pr = P + d.off;
-  double4* Fr = F + d.off;
+  const size_t T = st.total;   // stride between the components of a vector array
+  double* __restrict__ Rr = st.R + d.off;
+  double* __restrict__ Pr = st.P + d.off;
+  double* __restrict__ Fr = st.F + d.off;
+  double* __restrict__ Rs = st.Rsave + d.off;
+  double* __restrict__ Fs = st.Fsave + d.off;
+  uint4* __restrict__ qb = qbuild + d.off;
+  unsigned short* __restrict__ list = nlist + (size_t)d.off * cap;
   const double L = d.L, hdt = 0.5 * dt;
   const float c0 = 4.0f, c1 = 24.0f, c2 = 1.0f;   // pair_lj_cut with epsilon = sigma = 1
 
   // cell list of the current coordinates (fixed point in LDS)
-  auto count_of = [&](int c) { return (int)((ccount2[c >> 1] >> ((c & 1) * 16)) & 0xffffu); };
+  auto count_of = [&](int c) { return (int)((s.ccount2[c >> 1] >> ((c & 1) * 16)) & 0xffffu); };
   auto bump = [&](int c) {   // returns the previous count of cell c
-    unsigned int old = atomicAdd(&ccount2[c >> 1], 1u << ((c & 1) * 16));
+    unsigned int old = atomicAdd(&s.ccount2[c >> 1], 1u << ((c & 1) * 16));
     return (int)((old >> ((c & 1) * 16)) & 0xffffu);
   };
-  // fixed-point coordinates of the current R into LDS; returns the largest
-  // squared displacement since the last list build (scaled units^2)
-  auto refresh = [&]() -> double {
-    double m = 0.0;
-    for (int i = threadIdx.x; i < N; i += BS) {
-      double4 ri = Rr[i];
-      double s[3] = { ri.x / L, ri.y / L, ri.z / L };
-      unsigned int u[3];
-      for (int x = 0; x < 3; x++) {
-        double f = s[x] - floor(s[x]);
-        u[x] = (unsigned int)(unsigned long long)llrint(f * 4294967296.0);
-      }
-      qx[i] = u[0]; qy[i] = u[1]; qz[i] = u[2];
-      uint4 b = qbuild[d.off + i];
-      double ex = (double)(int)(u[0] - b.x), ey = (double)(int)(u[1] - b.y), ez = (double)(int)(u[2] - b.z);
-      m = fmax(m, (ex * ex + ey * ey + ez * ez) * (1.0 / 18446744073709551616.0));
+  // fixed-point coordinates of x (atom i) into LDS; returns the squared
+  // displacement since the last list build (scaled units^2)
+  auto place = [&](int i, const double (&x)[3]) __attribute__((always_inline)) {
+    unsigned int u[3];
+    for (int c = 0; c < 3; c++) {
+      double v = x[c] / L, f = v - floor(v);
+      u[c] = (unsigned int)(unsigned long long)llrint(f * 4294967296.0);
     }
+    s.qxy[i] = make_uint2(u[0], u[1]);
+    s.qz[i] = u[2];
+    uint4 b = qb[i];
+    double ex = (double)(int)(u[0] - b.x), ey = (double)(int)(u[1] - b.y), ez = (double)(int)(u[2] - b.z);
+    return (ex * ex + ey * ey + ez * ez) * (1.0 / 18446744073709551616.0);
+  };
+  auto block_max = [&](double m) {
     m = wave_max(m);
     int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     __syncthreads();
@@ -158,49 +187,53 @@ k_hmc(const ReplicaDesc* __restrict__ desc, const int* __restrict__ order, doubl
   // cell list of the coordinates in LDS, cells of side L / Mc
   auto build_cells = [&](int Mc) {
     const int ncc = Mc * Mc * Mc;
-    for (int c = threadIdx.x; c < (ncc + 1) / 2; c += BS) ccount2[c] = 0;
+    for (int c = threadIdx.x; c < (ncc + 1) / 2; c += BS) s.ccount2[c] = 0;
     __syncthreads();
     auto cell_of = [&](int i) {
-      return (int)(((unsigned long long)qx[i] * Mc) >> 32) +
-             Mc * ((int)(((unsigned long long)qy[i] * Mc) >> 32) + Mc * (int)(((unsigned long long)qz[i] * Mc) >> 32));
+      const uint2 xy = s.qxy[i];
+      return (int)(((unsigned long long)xy.x * Mc) >> 32) +
+             Mc * ((int)(((unsigned long long)xy.y * Mc) >> 32) + Mc * (int)(((unsigned long long)s.qz[i] * Mc) >> 32));
     };
     for (int i = threadIdx.x; i < N; i += BS) bump(cell_of(i));
     __syncthreads();
-    // exclusive scan of the counts: per-thread chunk sums, block scan, chunks
-    int chunk = (ncc + BS - 1) / BS, c0i = threadIdx.x * chunk, c1i = min(ncc, c0i + chunk);
+    // exclusive scan of the counts: per-thread chunk sums, a scan over the
+    // wave and over the waves' totals, chunks
+    int chunk = (ncc + BS - 1) / BS, c0i = min(ncc, (int)threadIdx.x * chunk), c1i = min(ncc, c0i + chunk);
     int local = 0;
     for (int c = c0i; c < c1i; c++) local += count_of(c);
-    scanTmp[threadIdx.x] = local;
-    __syncthreads();
-    for (int off = 1; off < BS; off <<= 1) {
-      int v = threadIdx.x >= off ? scanTmp[threadIdx.x - off] : 0;
-      __syncthreads();
-      scanTmp[threadIdx.x] += v;
-      __syncthreads();
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int incl = local;
+    for (int off = 1; off < 64; off <<= 1) {
+      int v = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += v;
     }
-    int run = scanTmp[threadIdx.x] - local;
-    for (int c = c0i; c < c1i; c++) { cstart[c] = run; run += count_of(c); }
-    if (threadIdx.x == 0) cstart[ncc] = N;
+    if (lane == 63) scanTmp[w] = incl;
     __syncthreads();
-    for (int c = threadIdx.x; c < (ncc + 1) / 2; c += BS) ccount2[c] = 0;
+    int run = incl - local;
+    for (int k = 0; k < w; k++) run += scanTmp[k];
+    for (int c = c0i; c < c1i; c++) { s.cstart[c] = (unsigned short)run; run += count_of(c); }
+    if (threadIdx.x == 0) s.cstart[ncc] = (unsigned short)N;
+    __syncthreads();
+    for (int c = threadIdx.x; c < (ncc + 1) / 2; c += BS) s.ccount2[c] = 0;
     __syncthreads();
     for (int i = threadIdx.x; i < N; i += BS) {
       int c = cell_of(i);
-      clist[cstart[c] + bump(c)] = (unsigned short)i;
+      s.clist[s.cstart[c] + bump(c)] = (unsigned short)i;
     }
     __syncthreads();
   };
-  // visits, for atom i, every atom j of the cells within Mc-cell reach that
-  // can lie within sqrt(R2s) (scaled units) of it, culled row by row; the
-  // atom itself is among them.  Mc < 2 DIV + 1: one cell holds every atom.
-  auto walk = [&](int i, int Mc, double R2s, auto&& visit) {
+  // gives visit, for atom i, the ranges of cell-sorted places (s.clist) of the
+  // cells within Mc-cell reach that can lie within sqrt(R2s) (scaled units) of
+  // it, culled row by row; the atom itself is among them.  Mc < 2 DIV + 1: one
+  // cell holds every atom.
+  auto walk = [&](int i, int Mc, double R2s, auto&& visit) __attribute__((always_inline)) {
     const int w = (Mc >= 2 * DIV + 1) ? DIV : 0;
     // cutoff^2 in cell units, with margins far above the FP32 rounding of the
     // culling (which can then only keep extra cells)
     const float rcell2 = (float)(R2s * (double)Mc * (double)Mc * (1.0 + 1e-5) + 1e-5);
-    unsigned int ui = qx[i], vi = qy[i], wi = qz[i];
-    unsigned long long px = (unsigned long long)ui * Mc, py = (unsigned long long)vi * Mc,
-                       pz = (unsigned long long)wi * Mc;
+    const uint2 xy = s.qxy[i];
+    unsigned long long px = (unsigned long long)xy.x * Mc, py = (unsigned long long)xy.y * Mc,
+                       pz = (unsigned long long)s.qz[i] * Mc;
     int cx = (int)(px >> 32), cy = (int)(py >> 32), cz = (int)(pz >> 32);
     // position of atom i inside its cell, in cell units
     const float ox = (float)(unsigned int)px * 2.3283064e-10f, oy = (float)(unsigned int)py * 2.3283064e-10f,
@@ -229,126 +262,149 @@ k_hmc(const ReplicaDesc* __restrict__ desc, const int* __restrict__ order, doubl
         for (int part = 0; part < 2; part++) {
           int ca = part == 0 ? r0a : r1a, cb = part == 0 ? r0b : r1b;
           if (cb < ca) continue;
-          int t0 = (w == 0) ? 0 : cstart[base + ca], t1 = (w == 0) ? N : cstart[base + cb + 1];
-          for (int t = t0; t < t1; t++) visit((w == 0) ? t : (int)clist[t]);
+          visit((w == 0) ? 0 : (int)s.cstart[base + ca], (w == 0) ? N : (int)s.cstart[base + cb + 1]);
         }
       }
     }
   };
   // Verlet list at radius sqrt(d.Rl2s) from the coordinates in LDS (every
   // atom within it, in walk order; the FP32 test keeps a margin, so the list
-  // may hold a few more); the build coordinates are kept for the trigger
+  // may hold a few more); the build coordinates are kept for the trigger.
+  // Entry n of atom i is 8 j at list[8 ((n/8) N + i) + n%8]; four entries are
+  // gathered in a register pair and stored together, and the last packet is
+  // padded with the atom itself.
+  // Measured (same replicas): one 16-bit store per entry 4.00 ms a cycle, this
+  // 3.82; atoms taken in cell order, whose lanes read the same candidates but
+  // store apart, 4.35; candidates read four at a time 4.48.
   auto build_list = [&]() {
     build_cells(d.Ml);
     const float rl2 = (float)(d.Rl2s * 18446744073709551616.0 * (1.0 + 1e-4));
     int over = 0;
     for (int i = threadIdx.x; i < N; i += BS) {
-      const unsigned int ui = qx[i], vi = qy[i], wi = qz[i];
+      const uint2 xy = s.qxy[i];
+      const unsigned int wi = s.qz[i];
       int n = 0;
-      walk(i, d.Ml, d.Rl2s, [&](int j) {
-        float ddx = (float)(int)(ui - qx[j]), ddy = (float)(int)(vi - qy[j]), ddz = (float)(int)(wi - qz[j]);
-        float r2 = ddx * ddx + ddy * ddy + ddz * ddz;
-        if (r2 < rl2 && j != i) {
-          if (n < cap) nlist[(size_t)d.off * cap + (size_t)n * N + i] = (unsigned short)j;
-          n++;
+      unsigned int lo = 0, hi = 0;   // the last four entries, the oldest lowest
+      unsigned short* __restrict__ li = list + 8 * (size_t)i;
+      auto put = [&](int j) __attribute__((always_inline)) {
+        lo = __builtin_amdgcn_alignbit(hi, lo, 16);
+        hi = __builtin_amdgcn_alignbit((unsigned int)(8 * j), hi, 16);
+        if ((n & 3) == 3 && n < cap)
+          *reinterpret_cast<uint2*>(li + 8 * (size_t)(n >> 3) * N + (n & 4)) = make_uint2(lo, hi);
+        n++;
+      };
+      walk(i, d.Ml, d.Rl2s, [&](int a, int b) __attribute__((always_inline)) {
+        for (int q = a; q < b; q++) {
+          const int j = s.clist[q];
+          const uint2 v = s.qxy[j];
+          float ddx = (float)(int)(xy.x - v.x), ddy = (float)(int)(xy.y - v.y), ddz = (float)(int)(wi - s.qz[j]);
+          float r2 = ddx * ddx + ddy * ddy + ddz * ddz;
+          if (r2 < rl2 && j != i) put(j);
         }
       });
-      nnb[d.off + i] = (unsigned short)min(n, cap);
-      qbuild[d.off + i] = make_uint4(ui, vi, wi, 0u);
-      over |= n > cap;
+      const int cnt = n;
+      while (n & 7) put(i);
+      nnb[d.off + i] = (unsigned short)min(cnt, cap);
+      qb[i] = make_uint4(xy.x, xy.y, wi, 0u);
+      over |= cnt > cap;
     }
-    // any overflow: this replica walks the cells from now on
+    // any overflow: this replica takes every atom from now on
     over = __syncthreads_or(over);
     if (threadIdx.x == 0) listState = over ? 2 : 1;
     __syncthreads();
   };
 
-  // forces F = -dU/dR and, with E_ true, the potential energy of the replica
-  // (only the last step of a trajectory needs it)
-  auto forces = [&](auto E_) -> double {
+  // force on atom i from its partners, and with E_ true its pair energies
+  auto force_of = [&](int i, bool useList, auto E_, double (&f)[3], double& ei) __attribute__((always_inline)) {
     constexpr bool WANT_E = decltype(E_)::value;
-    // the list: rebuilt when it is missing or an atom moved more than skin/2
-    const double moved = refresh();
-    if (listState != 2 && (listState == 0 || moved > d.trig2s)) build_list();
-    const bool useList = listState == 1;
-    double e = 0.0;
-    for (int i = threadIdx.x; i < N; i += BS) {
-      const unsigned int ui = qx[i], vi = qy[i], wi = qz[i];
-      double4 ri = Rr[i];
-      double fx = 0, fy = 0, fz = 0, ei = 0;
-      auto pair = [&](int j) {
-        if (MIXED) {
-          // the atom itself (zero separation) is masked, not branched over
-          float ddx = (float)(int)(ui - qx[j]), ddy = (float)(int)(vi - qy[j]), ddz = (float)(int)(wi - qz[j]);
-          float r2 = ddx * ddx + ddy * ddy + ddz * ddz;
-          bool in = r2 < d.lo && j != i;
-          if (r2 >= d.lo && r2 < d.hi) {
-            double4 rj = Rr[j];
-            double ex = ri.x / L - rj.x / L, ey = ri.y / L - rj.y / L, ez = ri.z / L - rj.z / L;
-            ex = ex - rint(ex); ey = ey - rint(ey); ez = ez - rint(ez);
-            double q2;
-            {
-#pragma clang fp contract(off)
-              q2 = ex * ex + ey * ey + ez * ez;
-            }
-            in = q2 < d.Rc2s;
-          }
-          if (in) {
-            float invR2 = d.K * __builtin_amdgcn_rcpf(r2);
-            float sr2 = c2 * invR2, sr6 = sr2 * sr2 * sr2;
-            float W = c1 * sr6 * (sr6 + sr6 - 1.0f);
-            float g = W * invR2;
-            fx += (double)(g * ddx);
-            fy += (double)(g * ddy);
-            fz += (double)(g * ddz);
-            if (WANT_E) ei += (double)(c0 * sr6 * (sr6 - 1.0f));
-          }
-        } else {
-          if (j == i) return;
-          double4 rj = Rr[j];
-          double ex = ri.x / L - rj.x / L, ey = ri.y / L - rj.y / L, ez = ri.z / L - rj.z / L;
-          ex = ex - rint(ex); ey = ey - rint(ey); ez = ez - rint(ez);
-          double q2;
-          {
-#pragma clang fp contract(off)
-            q2 = ex * ex + ey * ey + ez * ez;
-          }
-          if (q2 < d.Rc2s) {
-            double invR2 = 1.0 / (L * L * q2);
-            double sr2 = invR2, sr6 = sr2 * sr2 * sr2, sr12 = sr6 * sr6;
-            double W = 24.0 * (sr12 + sr12 - sr6);
-            double g = W * invR2;
-            fx += g * ex;
-            fy += g * ey;
-            fz += g * ez;
-            if (WANT_E) ei += 4.0 * (sr12 - sr6);
-          }
+    const uint2 xy = s.qxy[i];
+    const unsigned int wi = s.qz[i], io = 8u * (unsigned int)i;
+    double fx = 0, fy = 0, fz = 0, e = 0;
+    double xi[3] = { 0, 0, 0 };
+    if (!MIXED) for (int c = 0; c < 3; c++) xi[c] = Rr[c * T + i];
+    // o: 8 j
+    auto pair = [&](unsigned int o) __attribute__((always_inline)) {
+      // the pair's r^2 in scaled units and its separation, in FP64
+      auto exact = [&](double (&q)[3]) {
+        const size_t j = o >> 3;
+        for (int c = 0; c < 3; c++) {
+          const double x = MIXED ? Rr[c * T + i] : xi[c];
+          q[c] = x / L - Rr[c * T + j] / L;
+          q[c] = q[c] - rint(q[c]);
         }
+        double q2;
+        {
+#pragma clang fp contract(off)
+          q2 = q[0] * q[0] + q[1] * q[1] + q[2] * q[2];
+        }
+        return q2;
       };
-      if (useList) {
-        // eight indices loaded before their pairs are evaluated, so that
-        // the loads overlap; past the list end the atom itself stands in,
-        // which the pair body skips (FP64) or masks (mixed), so the eight
-        // are evaluated without a branch
-        const unsigned short* __restrict__ li = nlist + (size_t)d.off * cap + i;
-        const int n = nnb[d.off + i];
-        for (int k = 0; k < n; k += 8) {
-          int jb[8];
-#pragma unroll
-          for (int u = 0; u < 8; u++) jb[u] = k + u < n ? (int)li[(size_t)(k + u) * N] : i;
-#pragma unroll
-          for (int u = 0; u < 8; u++) pair(jb[u]);
+      if (MIXED) {
+        // the atom itself (zero separation) is masked, not branched over
+        const uint2 v = *reinterpret_cast<const uint2*>(reinterpret_cast<const char*>(s.qxy) + o);
+        const unsigned int vz = *reinterpret_cast<const unsigned int*>(reinterpret_cast<const char*>(s.qz) + (o >> 1));
+        float ddx = (float)(int)(xy.x - v.x), ddy = (float)(int)(xy.y - v.y), ddz = (float)(int)(wi - vz);
+        float r2 = ddx * ddx + ddy * ddy + ddz * ddz;
+        bool in = r2 < d.lo && o != io;
+        if (r2 >= d.lo && r2 < d.hi) {
+          double q[3];
+          in = exact(q) < d.Rc2s;
+        }
+        if (in) {
+          float invR2 = d.K * __builtin_amdgcn_rcpf(r2);
+          float sr2 = c2 * invR2, sr6 = sr2 * sr2 * sr2;
+          float W = c1 * sr6 * (sr6 + sr6 - 1.0f);
+          float g = W * invR2;
+          fx += (double)(g * ddx);
+          fy += (double)(g * ddy);
+          fz += (double)(g * ddz);
+          if (WANT_E) e += (double)(c0 * sr6 * (sr6 - 1.0f));
         }
       } else {
-        // a list that would overflow its capacity (more neighbours within
-        // rc + skin than LJ atoms at close packing hold): every atom
-        for (int j = 0; j < N; j++) pair(j);
+        if (o == io) return;
+        double q[3];
+        const double q2 = exact(q);
+        if (q2 < d.Rc2s) {
+          double invR2 = 1.0 / (L * L * q2);
+          double sr2 = invR2, sr6 = sr2 * sr2 * sr2, sr12 = sr6 * sr6;
+          double W = 24.0 * (sr12 + sr12 - sr6);
+          double g = W * invR2;
+          fx += g * q[0];
+          fy += g * q[1];
+          fz += g * q[2];
+          if (WANT_E) e += 4.0 * (sr12 - sr6);
+        }
       }
-      double sc = MIXED ? d.unit : L;
-      Fr[i] = make_double4(sc * fx, sc * fy, sc * fz, 0.0);
-      e += ei;
+    };
+    if (useList) {
+      // packets of eight, the next one loaded before this one's pairs
+      const int np = ((int)nnb[d.off + i] + 7) >> 3;
+      const uint4* __restrict__ lp = reinterpret_cast<const uint4*>(list) + i;
+      uint4 nx = np > 0 ? lp[0] : make_uint4(0, 0, 0, 0);
+      for (int p = 0; p < np; p++) {
+        const uint4 c = nx;
+        if (p + 1 < np) nx = lp[(size_t)(p + 1) * N];
+        const unsigned int w[4] = { c.x, c.y, c.z, c.w };
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          pair(w[u] & 0xffffu);
+          pair(w[u] >> 16);
+        }
+      }
+    } else {
+      // a list that would overflow its capacity (more neighbours within
+      // rc + skin than LJ atoms at close packing hold): every atom
+      for (int j = 0; j < N; j++) pair(8u * (unsigned int)j);
     }
-    return WANT_E ? 0.5 * block_total<BS>(e, red) : 0.0;
+    const double sc = MIXED ? d.unit : L;
+    f[0] = sc * fx; f[1] = sc * fy; f[2] = sc * fz;
+    ei = e;
+  };
+  // the list for the coordinates in LDS: rebuilt when it is missing or an atom
+  // moved more than skin/2
+  auto check_list = [&](double moved) {
+    if (listState != 2 && (listState == 0 || moved > d.trig2s)) build_list();
+    return listState == 1;
   };
 
   // the list and its build coordinates persist between launches (written
@@ -356,8 +412,21 @@ k_hmc(const ReplicaDesc* __restrict__ desc, const int* __restrict__ order, doubl
   if (threadIdx.x == 0) listState = lstate[r];
   __syncthreads();
   if (mode == 0) {
-    double u = forces(std::true_type());
-    if (threadIdx.x == 0) { U[r] = u; lstate[r] = listState; }
+    double m = 0.0;
+    for (int i = threadIdx.x; i < N; i += BS) {
+      const double x[3] = { Rr[i], Rr[T + i], Rr[2 * T + i] };
+      m = fmax(m, place(i, x));
+    }
+    const bool useList = check_list(block_max(m));
+    double e = 0.0;
+    for (int i = threadIdx.x; i < N; i += BS) {
+      double f[3], ei;
+      force_of(i, useList, std::true_type(), f, ei);
+      for (int c = 0; c < 3; c++) Fr[c * T + i] = f[c];
+      e += ei;
+    }
+    e = 0.5 * block_total<BS>(e, red);
+    if (threadIdx.x == 0) { U[r] = e; lstate[r] = listState; }
     return;
   }
   const double sq = sqrt(d.kT);
@@ -367,49 +436,75 @@ k_hmc(const ReplicaDesc* __restrict__ desc, const int* __restrict__ order, doubl
   for (int cyc = 0; cyc < ncycles; cyc++) {
     const int cnum = cycleNow;
     const uint64_t stream = hmc_stream(r, cnum);
-    // momentum refresh (mass 1) and saved state
-    double k = 0.0;
+    // momentum refresh (mass 1), saved state, and the first half kick and drift
+    double k = 0.0, moved = 0.0;
     for (int i = threadIdx.x; i < N; i += BS) {
-      double n[3];
-      for (int x = 0; x < 3; x++) {
-        double u1 = hmc_uniform(seed, stream, 6ULL * i + 2 * x), u2 = hmc_uniform(seed, stream, 6ULL * i + 2 * x + 1);
-        n[x] = sq * (sqrt(-2.0 * log(u1)) * cos(TWO_PI_D * u2));
+      double x[3];
+      for (int c = 0; c < 3; c++) {
+        double u1 = hmc_uniform(seed, stream, 6ULL * i + 2 * c), u2 = hmc_uniform(seed, stream, 6ULL * i + 2 * c + 1);
+        double p = sq * (sqrt(-2.0 * log(u1)) * cos(TWO_PI_D * u2));
+        x[c] = Rr[c * T + i];
+        const double f = Fr[c * T + i];
+        Rs[c * T + i] = x[c];
+        Fs[c * T + i] = f;
+        k += p * p;
+        if (nsteps > 0) {
+          p = p + hdt * f;
+          x[c] = x[c] + dt * p;
+          Pr[c * T + i] = p;
+          Rr[c * T + i] = x[c];
+        }
       }
-      Pr[i] = make_double4(n[0], n[1], n[2], 0.0);
-      Rsave[d.off + i] = Rr[i];
-      Fsave[d.off + i] = Fr[i];
-      k += n[0] * n[0] + n[1] * n[1] + n[2] * n[2];
+      if (nsteps > 0) moved = fmax(moved, place(i, x));
     }
     const double U0 = Unow, H0 = U0 + 0.5 * block_total<BS>(k, red);
-    double U1 = U0;
-    for (int s = 0; s < nsteps; s++) {
-      for (int i = threadIdx.x; i < N; i += BS) {
-        double4 p = Pr[i], f = Fr[i], x = Rr[i];
-        p.x = p.x + hdt * f.x; p.y = p.y + hdt * f.y; p.z = p.z + hdt * f.z;
-        x.x = x.x + dt * p.x; x.y = x.y + dt * p.y; x.z = x.z + dt * p.z;
-        Pr[i] = p;
-        Rr[i] = x;
+    double U1 = U0, K1 = k;
+    for (int st = 0; st < nsteps; st++) {
+      const bool useList = check_list(block_max(moved));
+      if (st < nsteps - 1) {
+        // force, the end of this step and the first half kick of the next
+        for (int i = threadIdx.x; i < N; i += BS) {
+          double f[3], ei;
+          force_of(i, useList, std::false_type(), f, ei);
+          for (int c = 0; c < 3; c++) {
+            double p = Pr[c * T + i];
+            p = p + hdt * f[c];
+            p = p + hdt * f[c];
+            Pr[c * T + i] = p;
+          }
+        }
+        __syncthreads();   // every force of the old coordinates before any drift
+        moved = 0.0;
+        for (int i = threadIdx.x; i < N; i += BS) {
+          double x[3];
+          for (int c = 0; c < 3; c++) {
+            x[c] = Rr[c * T + i] + dt * Pr[c * T + i];
+            Rr[c * T + i] = x[c];
+          }
+          moved = fmax(moved, place(i, x));
+        }
+      } else {
+        double e = 0.0;
+        K1 = 0.0;
+        for (int i = threadIdx.x; i < N; i += BS) {
+          double f[3], ei, p[3];
+          force_of(i, useList, std::true_type(), f, ei);
+          for (int c = 0; c < 3; c++) {
+            Fr[c * T + i] = f[c];
+            p[c] = Pr[c * T + i] + hdt * f[c];
+          }
+          e += ei;
+          K1 += p[0] * p[0] + p[1] * p[1] + p[2] * p[2];
+        }
+        U1 = 0.5 * block_total<BS>(e, red);
       }
-      __syncthreads();
-      if (s == nsteps - 1) U1 = forces(std::true_type());
-      else forces(std::false_type());
-      for (int i = threadIdx.x; i < N; i += BS) {
-        double4 p = Pr[i], f = Fr[i];
-        p.x = p.x + hdt * f.x; p.y = p.y + hdt * f.y; p.z = p.z + hdt * f.z;
-        Pr[i] = p;
-      }
-      __syncthreads();
     }
-    k = 0.0;
-    for (int i = threadIdx.x; i < N; i += BS) {
-      double4 p = Pr[i];
-      k += p.x * p.x + p.y * p.y + p.z * p.z;
-    }
-    const double H1 = U1 + 0.5 * block_total<BS>(k, red);
+    const double H1 = U1 + 0.5 * block_total<BS>(K1, red);
     const double dH = H1 - H0;
     const bool accept = dH <= 0.0 || hmc_uniform(seed, stream, HMC_ACCEPT_COUNTER) < exp(-dH / d.kT);
     if (!accept)
-      for (int i = threadIdx.x; i < N; i += BS) { Rr[i] = Rsave[d.off + i]; Fr[i] = Fsave[d.off + i]; }
+      for (int i = threadIdx.x; i < N; i += BS)
+        for (int c = 0; c < 3; c++) { Rr[c * T + i] = Rs[c * T + i]; Fr[c * T + i] = Fs[c * T + i]; }
     __syncthreads();
     if (threadIdx.x == 0) {
       Unow = accept ? U1 : U0;
@@ -423,6 +518,13 @@ k_hmc(const ReplicaDesc* __restrict__ desc, const int* __restrict__ order, doubl
     __syncthreads();
   }
   if (threadIdx.x == 0) lstate[r] = listState;
+}
+
+// Coordinates of every replica as a host takes them, three values per atom.
+__global__ void k_hmc_coords(double* __restrict__ out, const double* __restrict__ R, size_t total) {
+  const size_t i = (size_t)blockIdx.x * BLOCK + threadIdx.x;
+  if (i < total)
+    for (int c = 0; c < 3; c++) out[3 * i + c] = R[c * total + i];
 }
 
 }  // namespace emdee
@@ -440,7 +542,8 @@ struct EmDeeHMC {
   std::vector<int> offsets, hN;
   DBuf<ReplicaDesc> desc;
   DBuf<int> order, cycle;
-  DBuf<double4> R, P, F, Rsave, Fsave;
+  DBuf<double> R, P, F, Rsave, Fsave;   // [3][total]
+  DBuf<double> coords;                  // [total][3], for EmDeeHMC_get
   DBuf<double> U, lastDH;
   DBuf<long long> accepted;
   int cap = 0;                   // Verlet-list entries per atom
@@ -455,9 +558,8 @@ struct EmDeeHMC {
 };
 
 namespace {
-using HmcKernel = void (*)(const ReplicaDesc*, const int*, double4*, double4*, double4*, double4*, double4*, double*,
-                           int*, long long*, double*, double, double, int, uint64_t, int, int, unsigned short*,
-                           unsigned short*, uint4*, int, int*, double*, int);
+using HmcKernel = void (*)(const ReplicaDesc*, const int*, HmcState, double*, int*, long long*, double*, double, int,
+                           uint64_t, int, int, unsigned short*, unsigned short*, uint4*, int, int*, double*, int);
 struct Variant { int bs, div; HmcKernel mixed, plain; };
 const Variant VARIANTS[] = {
   { 256, 1, k_hmc<256, 1, true>, k_hmc<256, 1, false> },
@@ -490,10 +592,10 @@ void set_cells(EmDeeHMC* h, int div) {
 void launch(EmDeeHMC* h, int v, int ncycles, int mode) {
   const Variant& var = VARIANTS[v];
   HmcKernel k = h->precision ? var.mixed : var.plain;
-  hipLaunchKernelGGL(k, dim3(h->nrep), dim3(var.bs), 0, h->stream, h->desc.p, h->order.p, h->R.p, h->P.p, h->F.p,
-                     h->Rsave.p, h->Fsave.p, h->U.p, h->cycle.p, h->accepted.p, h->lastDH.p, h->rc, h->dt, h->nsteps,
-                     h->seed, ncycles, mode, h->nlist.p, h->nnb.p, h->qbuild.p, h->cap, h->lstate.p, h->Uhist.p,
-                     HMC_HIST);
+  const HmcState st{ h->R.p, h->P.p, h->F.p, h->Rsave.p, h->Fsave.p, (size_t)h->total };
+  hipLaunchKernelGGL(k, dim3(h->nrep), dim3(var.bs), 0, h->stream, h->desc.p, h->order.p, st, h->U.p, h->cycle.p,
+                     h->accepted.p, h->lastDH.p, h->dt, h->nsteps, h->seed, ncycles, mode, h->nlist.p, h->nnb.p,
+                     h->qbuild.p, h->cap, h->lstate.p, h->Uhist.p, HMC_HIST);
   launch_check("hmc");
 }
 }  // namespace
@@ -532,8 +634,8 @@ EmDeeHMC* EmDeeHMC_create(int nrep, const int* natoms, const double* box, const 
   }
   h->total = off;
   // list capacity: 1.6 times the mean count at the densest replica's
-  // density, plus room for fluctuations (a replica that overflows walks its
-  // cells instead)
+  // density, plus room for fluctuations (a replica that overflows takes
+  // every atom instead), in whole packets of eight
   {
     double rho = 0.0, rl = rc + HMC_SKIN;
     for (int r = 0; r < nrep; r++) rho = std::max(rho, natoms[r] / (box[r] * box[r] * box[r]));
@@ -546,12 +648,12 @@ EmDeeHMC* EmDeeHMC_create(int nrep, const int* natoms, const double* box, const 
   std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return natoms[a] > natoms[b]; });
   h->desc.alloc(nrep); h->order.alloc(nrep); h->cycle.alloc(nrep); h->U.alloc(nrep); h->lastDH.alloc(nrep);
   h->accepted.alloc(nrep);
-  for (DBuf<double4>* b : { &h->R, &h->P, &h->F, &h->Rsave, &h->Fsave }) b->alloc(off);
+  for (DBuf<double>* b : { &h->R, &h->P, &h->F, &h->Rsave, &h->Fsave }) b->alloc(3 * (size_t)off);
   h->nlist.alloc((size_t)off * h->cap); h->nnb.alloc(off); h->qbuild.alloc(off); h->lstate.alloc(nrep);
   h->Uhist.alloc((size_t)HMC_HIST * nrep);
-  std::vector<double4> R4(off);
-  for (int i = 0; i < off; i++) R4[i] = make_double4(R[3 * i], R[3 * i + 1], R[3 * i + 2], 0.0);
-  HIP_CHECK(hipMemcpy(h->R.p, R4.data(), sizeof(double4) * off, hipMemcpyHostToDevice));
+  std::vector<double> Rc(3 * (size_t)off);
+  for (int i = 0; i < off; i++) for (int c = 0; c < 3; c++) Rc[(size_t)c * off + i] = R[3 * (size_t)i + c];
+  HIP_CHECK(hipMemcpy(h->R.p, Rc.data(), sizeof(double) * Rc.size(), hipMemcpyHostToDevice));
   HIP_CHECK(hipMemcpy(h->order.p, ord.data(), sizeof(int) * nrep, hipMemcpyHostToDevice));
   std::vector<int> zeroI(nrep, 0);
   std::vector<long long> zeroL(nrep, 0);
@@ -572,13 +674,13 @@ EmDeeHMC* EmDeeHMC_create(int nrep, const int* natoms, const double* box, const 
 // division) from the same state, restores the state, and keeps the fastest.
 int EmDeeHMC_tune(EmDeeHMC* h) {
   int n = h->total, nr = h->nrep;
-  DBuf<double4> R0, F0;
+  DBuf<double> R0, F0;
   DBuf<double> U0;
   DBuf<int> c0;
   DBuf<long long> a0;
-  R0.alloc(n); F0.alloc(n); U0.alloc(nr); c0.alloc(nr); a0.alloc(nr);
-  HIP_CHECK(hipMemcpyAsync(R0.p, h->R.p, sizeof(double4) * n, hipMemcpyDeviceToDevice, h->stream));
-  HIP_CHECK(hipMemcpyAsync(F0.p, h->F.p, sizeof(double4) * n, hipMemcpyDeviceToDevice, h->stream));
+  R0.alloc(3 * (size_t)n); F0.alloc(3 * (size_t)n); U0.alloc(nr); c0.alloc(nr); a0.alloc(nr);
+  HIP_CHECK(hipMemcpyAsync(R0.p, h->R.p, 3 * sizeof(double) * n, hipMemcpyDeviceToDevice, h->stream));
+  HIP_CHECK(hipMemcpyAsync(F0.p, h->F.p, 3 * sizeof(double) * n, hipMemcpyDeviceToDevice, h->stream));
   HIP_CHECK(hipMemcpyAsync(U0.p, h->U.p, sizeof(double) * nr, hipMemcpyDeviceToDevice, h->stream));
   HIP_CHECK(hipMemcpyAsync(c0.p, h->cycle.p, sizeof(int) * nr, hipMemcpyDeviceToDevice, h->stream));
   HIP_CHECK(hipMemcpyAsync(a0.p, h->accepted.p, sizeof(long long) * nr, hipMemcpyDeviceToDevice, h->stream));
@@ -599,8 +701,8 @@ int EmDeeHMC_tune(EmDeeHMC* h) {
     HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
     h->tuneMs[v] = ms;
     if (ms < bestMs) { bestMs = ms; best = v; }
-    HIP_CHECK(hipMemcpyAsync(h->R.p, R0.p, sizeof(double4) * n, hipMemcpyDeviceToDevice, h->stream));
-    HIP_CHECK(hipMemcpyAsync(h->F.p, F0.p, sizeof(double4) * n, hipMemcpyDeviceToDevice, h->stream));
+    HIP_CHECK(hipMemcpyAsync(h->R.p, R0.p, 3 * sizeof(double) * n, hipMemcpyDeviceToDevice, h->stream));
+    HIP_CHECK(hipMemcpyAsync(h->F.p, F0.p, 3 * sizeof(double) * n, hipMemcpyDeviceToDevice, h->stream));
     HIP_CHECK(hipMemcpyAsync(h->U.p, U0.p, sizeof(double) * nr, hipMemcpyDeviceToDevice, h->stream));
     HIP_CHECK(hipMemcpyAsync(h->cycle.p, c0.p, sizeof(int) * nr, hipMemcpyDeviceToDevice, h->stream));
     HIP_CHECK(hipMemcpyAsync(h->accepted.p, a0.p, sizeof(long long) * nr, hipMemcpyDeviceToDevice, h->stream));
@@ -639,9 +741,12 @@ void EmDeeHMC_synchronize(EmDeeHMC* h) { HIP_CHECK(hipStreamSynchronize(h->strea
 void EmDeeHMC_get(EmDeeHMC* h, double* R, double* U, long long* accepted, double* lastDH) {
   HIP_CHECK(hipStreamSynchronize(h->stream));
   if (R) {
-    std::vector<double4> R4(h->total);
-    HIP_CHECK(hipMemcpy(R4.data(), h->R.p, sizeof(double4) * h->total, hipMemcpyDeviceToHost));
-    for (int i = 0; i < h->total; i++) { R[3 * i] = R4[i].x; R[3 * i + 1] = R4[i].y; R[3 * i + 2] = R4[i].z; }
+    h->coords.alloc(3 * (size_t)h->total);
+    hipLaunchKernelGGL(k_hmc_coords, dim3(div_up(h->total, BLOCK)), dim3(BLOCK), 0, h->stream, h->coords.p, h->R.p,
+                       (size_t)h->total);
+    launch_check("hmc coordinates");
+    HIP_CHECK(hipMemcpyAsync(R, h->coords.p, 3 * sizeof(double) * h->total, hipMemcpyDeviceToHost, h->stream));
+    HIP_CHECK(hipStreamSynchronize(h->stream));
   }
   if (U) HIP_CHECK(hipMemcpy(U, h->U.p, sizeof(double) * h->nrep, hipMemcpyDeviceToHost));
   if (accepted) HIP_CHECK(hipMemcpy(accepted, h->accepted.p, sizeof(long long) * h->nrep, hipMemcpyDeviceToHost));
@@ -680,7 +785,7 @@ void EmDeeHMC_destroy(EmDeeHMC* h) {
   if (h->exec) (void)hipGraphExecDestroy(h->exec);
   if (h->graph) (void)hipGraphDestroy(h->graph);
   h->desc.release(); h->order.release(); h->cycle.release(); h->U.release(); h->lastDH.release(); h->accepted.release();
-  for (DBuf<double4>* b : { &h->R, &h->P, &h->F, &h->Rsave, &h->Fsave }) b->release();
+  for (DBuf<double>* b : { &h->R, &h->P, &h->F, &h->Rsave, &h->Fsave, &h->coords }) b->release();
   h->nlist.release(); h->nnb.release(); h->qbuild.release(); h->lstate.release(); h->Uhist.release();
   (void)hipStreamDestroy(h->stream);
   delete h;
