@@ -140,9 +140,9 @@ struct Scaled {
   const int* charged;
   double L;
 };
-__device__ __forceinline__ void scale_vals(const Scaled& sc, double x, double y, double z, int s) {
-  double v[3] = { x / sc.L, y / sc.L, z / sc.L };
-  int t = sc.type[s];
+__device__ __forceinline__ void scale_vals(const Scaled& sc, double x, double y, double z, int s, int t, bool charged,
+                                           double charge, double (&v)[3], int4& q4) {
+  v[0] = x / sc.L; v[1] = y / sc.L; v[2] = z / sc.L;
   if (sc.Rs4) sc.Rs4[s] = make_double4(v[0], v[1], v[2], (double)t);
   if (sc.Q4) {
     unsigned int u[3];
@@ -151,9 +151,16 @@ __device__ __forceinline__ void scale_vals(const Scaled& sc, double x, double y,
       u[x] = (unsigned int)(unsigned long long)llrint(f * 4294967296.0);
     }
     bool fin = isfinite(v[0]) && isfinite(v[1]) && isfinite(v[2]);
-    sc.Q4[s] = make_int4((int)u[0], (int)u[1], (int)u[2], fin ? t : (t | Q4_NONFINITE));
-    if (sc.qf) sc.qf[s] = sc.charged[s] ? (float)sc.charge[s] : 0.0f;
+    q4 = make_int4((int)u[0], (int)u[1], (int)u[2], fin ? t : (t | Q4_NONFINITE));
+    sc.Q4[s] = q4;
+    if (sc.qf) sc.qf[s] = charged ? (float)charge : 0.0f;
   }
+}
+__device__ __forceinline__ void scale_vals(const Scaled& sc, double x, double y, double z, int s) {
+  double v[3];
+  int4 q4;
+  const bool q = sc.Q4 && sc.qf && sc.charged[s];
+  scale_vals(sc, x, y, z, s, sc.type[s], q, q ? sc.charge[s] : 0.0, v, q4);
 }
 __device__ __forceinline__ void scale_slot(const Scaled& sc, const double* __restrict__ R, int s, int Npad) {
   scale_vals(sc, R[s], R[Npad + s], R[2 * Npad + s], s);
@@ -338,12 +345,14 @@ __global__ void k_scan_add(int* __restrict__ out, const int* __restrict__ bsum, 
   int i = blockIdx.x * BLOCK + threadIdx.x;
   if (i < n) out[i] += bsum[blockIdx.x];
 }
-__global__ void k_cell_scatter(int* __restrict__ order, int* __restrict__ fill, const int* __restrict__ key,
+// Places every slot in its cell's range, in any order; takes each cell's count
+// back to zero, as the next sort needs it.
+__global__ void k_cell_scatter(int* __restrict__ order, int* __restrict__ count, const int* __restrict__ key,
                                const int* __restrict__ start, int N) {
   int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= N) return;
   int c = key[s];
-  order[start[c] + atomicAdd(&fill[c], 1)] = s;
+  order[start[c] + atomicSub(&count[c], 1) - 1] = s;
 }
 // Deterministic order inside each cell: ascending original atom index.  Each
 // entry of the scattered order counts the members of its cell with a smaller
@@ -358,12 +367,87 @@ __global__ void k_cell_rank(int* __restrict__ order, const int* __restrict__ sca
   for (int y = a; y < b; y++) rank += perm[scat[y]] < pv;
   order[a + rank] = v;
 }
-// ncomp consecutive [Npad] components at once
+// The whole sort in one workgroup: counts, scan, scatter and ranking in LDS,
+// to the same cellStart and order as the kernels above (a cell's members by
+// ascending original index).  Bound by the chain of its five passes over one
+// CU's LDS, which up to SORT_ATOMS atoms and SORT_CELLS cells costs less than
+// the launches (800 LJ atoms 4.3 us, 4,000 9.2; six kernels and two fills
+// 16 us of their own and 4 us between each).  Larger sorts have more atoms
+// than LDS.
+constexpr int SORT_ATOMS = 16384, SORT_CELLS = 16384, SORT_T = 1024;
+__global__ void __launch_bounds__(SORT_T)
+k_cell_sort_small(int* __restrict__ order, int* __restrict__ start, const double* __restrict__ R,
+                  const int* __restrict__ perm, const int* __restrict__ iperm, double L, int M, int N, int Npad) {
+  __shared__ int cnt[SORT_CELLS];               // counts, then starts, then ends
+  __shared__ unsigned short cell[SORT_ATOMS];   // of each slot
+  __shared__ unsigned short item[SORT_ATOMS];   // original indices, cell by cell
+  __shared__ int wsum[SORT_T / 64];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6, nc = M * M * M;
+  for (int c = t; c < nc; c += SORT_T) cnt[c] = 0;
+  __syncthreads();
+  for (int s = t; s < N; s += SORT_T) {
+    int ix = cell_coord(R[s] / L, M), iy = cell_coord(R[Npad + s] / L, M), iz = cell_coord(R[2 * Npad + s] / L, M);
+    int c = ix + M * (iy + M * iz);
+    cell[s] = (unsigned short)c;
+    atomicAdd(&cnt[c], 1);
+  }
+  __syncthreads();
+  // exclusive scan, an odd number of cells to a thread (no bank conflicts)
+  const int per = ((nc + SORT_T - 1) / SORT_T) | 1, a = min(t * per, nc), b = min(a + per, nc);
+  int sum = 0;
+  for (int c = a; c < b; c++) sum += cnt[c];
+  int incl = sum;
+  for (int off = 1; off < 64; off <<= 1) {
+    int y = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += y;
+  }
+  if (lane == 63) wsum[w] = incl;
+  __syncthreads();
+  int run = incl - sum;
+  for (int k = 0; k < w; k++) run += wsum[k];
+  for (int c = a; c < b; c++) {
+    int v = cnt[c];
+    cnt[c] = run;
+    run += v;
+  }
+  __syncthreads();
+  for (int c = t; c < nc; c += SORT_T) start[c] = cnt[c];
+  if (t == 0) start[nc] = N;
+  __syncthreads();
+  for (int s = t; s < N; s += SORT_T) item[atomicAdd(&cnt[cell[s]], 1)] = (unsigned short)perm[s];
+  __syncthreads();
+  for (int x = t; x < N; x += SORT_T) {
+    const int p = item[x], v = iperm[p], c = cell[v], f = c ? cnt[c - 1] : 0, e = cnt[c];
+    int rank = 0;
+    for (int y = f; y < e; y++) rank += item[y] < p;
+    order[f + rank] = v;
+  }
+}
+// Posts the list's entry count and the capacity it needs (0: it fits) to the
+// host, as k_reduce_post.
+__global__ void k_list_post(double* __restrict__ host, unsigned long long* __restrict__ hostSeq,
+                            unsigned long long seq, const double* __restrict__ partials, int nblocks,
+                            const int* __restrict__ flags) {
+  double v[1] = { 0 };
+#pragma unroll 8
+  for (int b = threadIdx.x; b < nblocks; b += BLOCK) v[0] += partials[b];
+  block_sum<1>(v);
+  if (threadIdx.x == 0) {
+    host[0] = v[0];
+    host[1] = (double)flags[0];
+    __threadfence_system();
+    *(volatile unsigned long long*)hostSeq = seq;
+  }
+}
 // Every per-slot array gathered into the new slot order in one pass: slot s
 // takes old slot order[s].  R goes to both R (via scratch) and R0 (the list's
 // reference positions); the inverse permutation is written as perm is.
 // F is permuted only when given (other layers' forces; the current layer's
-// are recomputed after every list build).
+// are recomputed after every list build).  The functions of R, type and charge
+// that the list build and the pair kernels read are formed on the way: the
+// scaled and fixed-point positions, the cell, and P16, the top 16 bits of each
+// fixed-point coordinate, x and y packed in one word, z with bit 31 set when
+// the position is not finite.  Clears the list build's overflow flag.
 struct PermuteAll {
   const int* order;
   const double *R, *P, *F, *invMass, *charge;
@@ -371,28 +455,43 @@ struct PermuteAll {
   const int *type, *body, *perm, *freeFlag, *chargedFlag;
   int *typen, *bodyn, *permn, *freeFlagn, *chargedFlagn, *iperm;
   int nF;
+  Scaled sc;
+  uint2* P16;
+  int *key, *flags;
+  int M;
 };
 __global__ void k_permute_all(PermuteAll a, int N, int Npad) {
   int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s == 0) a.flags[0] = 0;
   if (s >= N) return;
   const int o = a.order[s];
+  double x[3];
   for (int c = 0; c < 3; c++) {
     double r = a.R[(size_t)c * Npad + o];
+    x[c] = r;
     a.Rn[(size_t)c * Npad + s] = r;
     a.R0[(size_t)c * Npad + s] = r;
     a.Pn[(size_t)c * Npad + s] = a.P[(size_t)c * Npad + o];
   }
   if (a.F)
     for (int c = 0; c < a.nF; c++) a.Fn[(size_t)c * Npad + s] = a.F[(size_t)c * Npad + o];
+  const double q = a.charge[o];
+  const int t = a.type[o], charged = a.chargedFlag[o];
   a.invMassn[s] = a.invMass[o];
-  a.chargen[s] = a.charge[o];
-  a.typen[s] = a.type[o];
+  a.chargen[s] = q;
+  a.typen[s] = t;
   a.bodyn[s] = a.body[o];
   a.freeFlagn[s] = a.freeFlag[o];
-  a.chargedFlagn[s] = a.chargedFlag[o];
+  a.chargedFlagn[s] = charged;
   const int p = a.perm[o];
   a.permn[s] = p;
   a.iperm[p] = s;
+  double v[3];
+  int4 q4;
+  scale_vals(a.sc, x[0], x[1], x[2], s, t, charged != 0, q, v, q4);
+  a.key[s] = cell_coord(v[0], a.M) + a.M * (cell_coord(v[1], a.M) + a.M * cell_coord(v[2], a.M));
+  a.P16[s] = make_uint2(((unsigned int)q4.x >> 16) | ((unsigned int)q4.y & 0xffff0000u),
+                        ((unsigned int)q4.z >> 16) | ((q4.w & Q4_NONFINITE) ? 0x80000000u : 0u));
 }
 
 // ---- mixed form: FP32 pair arithmetic, FP64 accumulation -----------------
@@ -419,26 +518,13 @@ struct MixedCut {
   double L;
 };
 
-// P16 (optional): the top 16 bits of each fixed-point coordinate, x and y
-// packed in one word, z with bit 31 set when the position is not finite.
-// key (optional): the cell of each slot, as k_cell_key computes it.
 __global__ void k_scale4q(double4* __restrict__ Rs4, int4* __restrict__ Q4, float* __restrict__ qf,
                           const double* __restrict__ R, const int* __restrict__ type, const double* __restrict__ charge,
-                          const int* __restrict__ charged, double L, int N, int Npad, uint2* __restrict__ P16,
-                          int* __restrict__ key, int M) {
+                          const int* __restrict__ charged, double L, int N, int Npad) {
   int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= N) return;
   Scaled sc{ Rs4, Q4, qf, type, charge, charged, L };
   scale_slot(sc, R, s, Npad);
-  if (key) {
-    double4 r = Rs4[s];
-    key[s] = cell_coord(r.x, M) + M * (cell_coord(r.y, M) + M * cell_coord(r.z, M));
-  }
-  if (P16) {
-    int4 q = Q4[s];
-    P16[s] = make_uint2(((unsigned int)q.x >> 16) | ((unsigned int)q.y & 0xffff0000u),
-                        ((unsigned int)q.z >> 16) | ((q.w & Q4_NONFINITE) ? 0x80000000u : 0u));
-  }
 }
 
 // relative half-width of the FP32 band around a cutoff Rc2s (scaled units^2)
@@ -2223,6 +2309,7 @@ static void ensure_cells(Device* d, int M) {
   d->M = M;
   d->ncells = M * M * M;
   d->cellCount.alloc(d->ncells + 1);
+  HIP_CHECK(hipMemsetAsync(d->cellCount.p, 0, sizeof(int) * (d->ncells + 1), d->stream));
   d->cellStart.alloc(d->ncells + 1);
   d->blockSums.alloc(div_up(d->ncells + 1, BLOCK) + 1);
 }
@@ -2246,20 +2333,29 @@ void dev_rebuild(Device* d, double L, double xRc, double rc, bool mixed) {
   int nc = d->ncells, nc1 = nc + 1, gc = div_up(nc1, BLOCK);
   // counting sort by cell: count, exclusive scan over ncells+1 entries
   // (start[ncells] = N), scatter, order inside cells
-  HIP_CHECK(hipMemsetAsync(d->cellCount.p, 0, sizeof(int) * nc1, d->stream));
-  hipLaunchKernelGGL(k_cell_key, dim3(g), dim3(BLOCK), 0, d->stream, d->key.p, d->cellCount.p, d->R.p, L, M, N, Np);
-  hipLaunchKernelGGL(k_scan_block, dim3(gc), dim3(BLOCK), 0, d->stream, d->cellStart.p, d->blockSums.p, d->cellCount.p, nc1);
-  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_T), 0, d->stream, d->blockSums.p, gc, (int*)nullptr);
-  hipLaunchKernelGGL(k_scan_add, dim3(gc), dim3(BLOCK), 0, d->stream, d->cellStart.p, d->blockSums.p, nc1);
-  HIP_CHECK(hipMemsetAsync(d->cellCount.p, 0, sizeof(int) * nc1, d->stream));
-  // scattered (in-cell order of the atomics) into tmpI, which is free until
-  // the permutation below, then ranked into order
-  hipLaunchKernelGGL(k_cell_scatter, dim3(g), dim3(BLOCK), 0, d->stream, d->tmpI.p, d->cellCount.p, d->key.p, d->cellStart.p, N);
-  hipLaunchKernelGGL(k_cell_rank, dim3(g), dim3(BLOCK), 0, d->stream, d->order.p, d->tmpI.p, d->key.p, d->cellStart.p,
-                     d->perm.p, N);
+  if (N <= SORT_ATOMS && nc <= SORT_CELLS) {
+    hipLaunchKernelGGL(k_cell_sort_small, dim3(1), dim3(SORT_T), 0, d->stream, d->order.p, d->cellStart.p, d->R.p,
+                       d->perm.p, d->iperm.p, L, M, N, Np);
+  } else {
+    hipLaunchKernelGGL(k_cell_key, dim3(g), dim3(BLOCK), 0, d->stream, d->key.p, d->cellCount.p, d->R.p, L, M, N, Np);
+    hipLaunchKernelGGL(k_scan_block, dim3(gc), dim3(BLOCK), 0, d->stream, d->cellStart.p, d->blockSums.p, d->cellCount.p,
+                       nc1);
+    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_T), 0, d->stream, d->blockSums.p, gc, (int*)nullptr);
+    hipLaunchKernelGGL(k_scan_add, dim3(gc), dim3(BLOCK), 0, d->stream, d->cellStart.p, d->blockSums.p, nc1);
+    // scattered (in-cell order of the atomics) into tmpI, which is free until
+    // the permutation below, then ranked into order
+    hipLaunchKernelGGL(k_cell_scatter, dim3(g), dim3(BLOCK), 0, d->stream, d->tmpI.p, d->cellCount.p, d->key.p,
+                       d->cellStart.p, N);
+    hipLaunchKernelGGL(k_cell_rank, dim3(g), dim3(BLOCK), 0, d->stream, d->order.p, d->tmpI.p, d->key.p, d->cellStart.p,
+                       d->perm.p, N);
+  }
   launch_check("cell sort");
   // every per-slot array into the new order (written to scratch, swapped),
-  // R0 = R, and the inverse permutation
+  // R0 = R, the inverse permutation, and the scaled and fixed-point positions
+  // and cells in the new order
+  d->Q4.alloc(Np);
+  d->qf.alloc(Np);
+  d->P16.alloc(Np + 16);               // the segment list build reads up to 16 slots past N
   {
     PermuteAll pa;
     pa.order = d->order.p;
@@ -2274,6 +2370,8 @@ void dev_rebuild(Device* d, double L, double xRc, double rc, bool mixed) {
     pa.freeFlag = d->freeFlag.p; pa.freeFlagn = d->tmpFree.p;
     pa.chargedFlag = d->chargedFlag.p; pa.chargedFlagn = d->tmpCharged.p;
     pa.iperm = d->iperm.p;
+    pa.sc = Scaled{ d->Rs4.p, d->Q4.p, d->qf.p, nullptr, nullptr, nullptr, L };
+    pa.P16 = d->P16.p; pa.key = d->key.p; pa.flags = d->flags.p; pa.M = M;
     hipLaunchKernelGGL(k_permute_all, dim3(g), dim3(BLOCK), 0, d->stream, pa, N, Np);
     auto swapD = [](DBuf<double>& x, DBuf<double>& y) { std::swap(x.p, y.p); std::swap(x.n, y.n); };
     auto swapI = [](DBuf<int>& x, DBuf<int>& y) { std::swap(x.p, y.p); std::swap(x.n, y.n); };
@@ -2283,13 +2381,6 @@ void dev_rebuild(Device* d, double L, double xRc, double rc, bool mixed) {
     swapI(d->freeFlag, d->tmpFree); swapI(d->chargedFlag, d->tmpCharged);
   }
   launch_check("permute");
-  // scaled and fixed-point positions and keys in the new order (functions of
-  // R, type and charge)
-  d->Q4.alloc(Np);
-  d->qf.alloc(Np);
-  d->P16.alloc(Np + 16);               // the segment list build reads up to 16 slots past N
-  hipLaunchKernelGGL(k_scale4q, dim3(g), dim3(BLOCK), 0, d->stream, d->Rs4.p, d->Q4.p, d->qf.p, d->R.p, d->type.p,
-                     d->charge.p, d->chargedFlag.p, L, N, Np, d->P16.p, d->key.p, M);
 
   // Verlet list, growing the ELL capacity on overflow
   double xRc2 = (xRc * xRc) / (L * L);
@@ -2311,7 +2402,6 @@ void dev_rebuild(Device* d, double L, double xRc, double rc, bool mixed) {
   }
   for (;;) {
     d->nbr.alloc((size_t)d->cap * Np);
-    HIP_CHECK(hipMemsetAsync(d->flags.p, 0, sizeof(int) * 4, d->stream));
     int gl = div_up((long)N * S, BLOCK);
     hipEvent_t e0 = d->profiling ? d->ev0 : nullptr, e1 = d->profiling ? d->ev1 : nullptr;
     // the segment-streaming form addresses list entries with 32-bit element
@@ -2336,19 +2426,22 @@ void dev_rebuild(Device* d, double L, double xRc, double rc, bool mixed) {
                             (const int4*)d->Q4.p, lo, hi, d->nsh.p, edge);
     }
     launch_check("build_list");
-    hipLaunchKernelGGL(k_reduce_partials<1>, dim3(1), dim3(BLOCK), 0, d->stream, d->result.p + 8, d->partials.p, gl);
-    HIP_CHECK(hipMemcpyAsync(d->hresult + 8, d->result.p + 8, sizeof(double), hipMemcpyDeviceToHost, d->stream));
-    int* hf = reinterpret_cast<int*>(d->hresult + 16);
-    HIP_CHECK(hipMemcpyAsync(hf, d->flags.p, sizeof(int), hipMemcpyDeviceToHost, d->stream));
-    HIP_CHECK(hipStreamSynchronize(d->stream));
+    const unsigned long long seq = ++d->seq;
+    hipLaunchKernelGGL(k_list_post, dim3(1), dim3(BLOCK), 0, d->stream, d->hpostDev + POST_LIST, d->hseqDev, seq,
+                       d->partials.p, gl, (const int*)d->flags.p);
+    launch_check("list totals");
+    post_wait(d, seq);
     if (d->profiling) {
+      HIP_CHECK(hipEventSynchronize(d->ev1));
       float ms = 0; HIP_CHECK(hipEventElapsedTime(&ms, d->ev0, d->ev1));
       d->listMs += ms; d->listLaunches++;
     }
-    if (hf[0] == 0) break;
-    d->cap = ((int)(hf[0] * 1.2) + 15) & ~7;
+    const int need = (int)d->hpost[POST_LIST + 1];
+    if (need == 0) break;
+    d->cap = ((int)(need * 1.2) + 15) & ~7;
+    HIP_CHECK(hipMemsetAsync(d->flags.p, 0, sizeof(int) * 4, d->stream));
   }
-  d->listEntries = d->hresult[8];
+  d->listEntries = d->hpost[POST_LIST];
   d->built = true;
   d->listVersion++;
 }
@@ -2384,7 +2477,7 @@ void dev_compute_pairs(Device* d, const PairCall& c, ForceSums* out) {
     d->Q4.alloc(Np);
     d->qf.alloc(Np);
     hipLaunchKernelGGL(k_scale4q, dim3(g), dim3(BLOCK), 0, d->stream, d->Rs4.p, d->Q4.p, d->qf.p, d->R.p, d->type.p,
-                       d->charge.p, d->chargedFlag.p, c.L, N, Np, (uint2*)nullptr, (int*)nullptr, 0);
+                       d->charge.p, d->chargedFlag.p, c.L, N, Np);
   } else {
     hipLaunchKernelGGL(k_scale4, dim3(g), dim3(BLOCK), 0, d->stream, d->Rs4.p, d->R.p, d->type.p, c.L, N, Np);
   }

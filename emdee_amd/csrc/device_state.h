@@ -196,10 +196,10 @@ __device__ __forceinline__ void finish_sums(const Post& post, double* __restrict
 // Slots in the posted-results block (64 doubles): the pair sums, the Ewald
 // energy and virial, the learned model's energy, virial and overflow flag,
 // the rigid bodies' kinetic-energy terms and their virial, the model's
-// low-k energy and virial, the rebuild trigger; the kick's kinetic energy uses
-// slot 0.
+// low-k energy and virial, the rebuild trigger, the list's entry count and
+// overflow flag; the kick's kinetic energy uses slot 0.
 constexpr int POST_PAIRS = 8, POST_EWALD = 16, POST_MODEL = 24, POST_BODY_KE = 32, POST_BODY_W = 40, POST_LOWK = 48,
-              POST_TRIG = 56;
+              POST_TRIG = 56, POST_LIST = 60;
 // Tickets of the kernels that finish their own sums
 enum { TICKET_KE, TICKET_TRIG, TICKET_BODY_KE, TICKET_BODY_W, TICKETS };
 
