@@ -847,7 +847,7 @@ k_build_list(int* __restrict__ nbr, int* __restrict__ nnb, int* __restrict__ fla
       settle();
       // one step ahead: the next step's position and body are loaded before
       // this step is tested (a lane without a candidate loads its own atom's)
-      // (32-bit offsets from the array bases: slots are below 2^21 here)
+      // (32-bit offsets from the array bases: slots are below 2^26 here)
       auto q4At = [&](int k) { return *(const int4*)((const char*)Q4 + (unsigned)k * 16u); };
       auto bodyAt = [&](int k) { return *(const int*)((const char*)body + (unsigned)k * 4u); };
       bool has = s < nseg;
@@ -2319,13 +2319,20 @@ void dev_rebuild(Device* d, double L, double xRc, double rc, bool mixed) {
   if (N == 0) return;
   d->posWrites++;                      // R and R0 in a new slot order
   int g = div_up(N, BLOCK);
-  // lanes per atom of the list build: as many as keep at most 2^21 lanes in
-  // all and at least four candidates per lane (the scanned region is ~2.6
-  // times the list volume)
+  // lanes per atom of the list build.  Long lists (the scanned region is ~2.6
+  // times the list volume; four candidates per lane): 16, whose streamed scan
+  // beats the row scans of 4 lanes or 1 at every size (196,608 water
+  // atoms, 4 lanes: 876 us, 16: 527; 600,000, 1 lane: 5.3 ms, 16: 1.6;
+  // 150,001 LJ atoms, 4 lanes: 153 us, 16: 93), except that the segment form is faster for simple systems of more than 2^19 atoms
+  // (600,000: 235 us for 322).  It is at 150,001 too (90 us for 93; 262,144:
+  // 107 for 150), but it lists band candidates last, and up to 2^19 atoms lists
+  // keep the scan order that their mixed sums have always followed.
+  // Short lists: 4 lanes up to 2^21 lanes in all.
   double vol = 4.18879020478639 * xRc * xRc * xRc * ((double)N / (L * L * L));   // expected list length
   const bool simple = d->bodies.nb == 0 && d->nexcl == 0 && d->allInteract;
   const double cand = 2.6 * vol;
-  const int S = (cand >= 16 * 4 && (long)N * 16 <= (1L << 21)) ? 16 : ((cand >= 4 * 4 && (long)N * 4 <= (1L << 21)) ? 4 : 1);
+  const bool small = (long)N * 4 <= (1L << 21);
+  const int S = (cand >= 16 * 4 && (small || !simple) && N < (1 << 26)) ? 16 : ((cand >= 4 * 4 && small) ? 4 : 1);
   int M = (int)std::floor(CELL_REACH * L / xRc);
   if (M < 2 * CELL_REACH + 1) M = 2 * CELL_REACH + 1;   // every cell of a row at most once
   if ((long)M * M * M > 64l * 1024 * 1024) M = 400;   // bound the cell table
