@@ -713,12 +713,11 @@ __device__ __forceinline__ void scan_range(int a, int b, int i, double xi, doubl
 // a scan over the lanes that places all four parts at once: 444 us.)
 // Where the order changes, so does the rounding of the sums.  Lists for the
 // mixed form keep the scan order: its FP32 sums of four entries follow the
-// list.  So do systems of more than SHELL_ATOMS atoms, though 98,304 would gain
-// (pair kernel 398 -> 314 us, build 269 -> 353 us): among so many molecules a
-// few amplify a rounding so fast that momenta moved by 4e-8 within 20 steps of
-// 2 fs, where every other change of order stays below 1e-9.
+// list, and would move results by 1e-6.  In FP64 momenta move by 1e-13 of
+// their size within 20 steps of 2 fs (98,304 water atoms, where a list build
+// goes from 269 to 353 us and the pair kernel from 398 to 314, ten steps from
+// 5.99 to 5.38 ms).
 constexpr int FAR_CAP = 300;   // 32 KB of LDS a block: five blocks per CU
-constexpr int SHELL_ATOMS = 16384;
 struct ShellCut {            // for the pair kernels
   const int4* nsh;           // null: lists without shells
   const double* trig;        // [0]: largest squared displacement since the build
@@ -2400,7 +2399,12 @@ void dev_rebuild(Device* d, double L, double xRc, double rc, bool mixed) {
     d->shellEdge[k] = e * (1.0 - 1e-5);
     (&edge.x)[k] = (float)(e * e / (L * L) * two32 * two32);
   }
-  d->shells = S == 16 && !mixed && N <= SHELL_ATOMS;
+  // shells for the multi-lane pair kernels.  A lane that walks its list alone
+  // gains less than the build loses: 150,001 LJ atoms, 20 steps 2.39 -> 2.45
+  // ms, 400,000: 4.75 -> 4.86 (with 16 lanes 30,000 and 60,000 are even)
+  bool lanes = N <= (1 << 16) || vol >= 96.0;   // as dev_compute_pairs has it
+  for (int l = 0; l < d->nlayers; l++) lanes = lanes && !lj_path(d, l);
+  d->shells = S == 16 && !mixed && lanes;
   d->listL = L;
   if (d->shells) d->nsh.alloc(Np);
   if (d->cap == 0) {
