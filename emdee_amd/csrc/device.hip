@@ -35,6 +35,7 @@
 #include "device_state.h"
 #include "engine.h"
 #include "pair_eval.h"
+#include "readback.h"
 
 namespace emdee {
 
@@ -92,6 +93,34 @@ __global__ void k_scatter_aos(double* __restrict__ aos, const double* __restrict
   aos[3 * o] = src[s];
   aos[3 * o + 1] = src[Npad + s];
   aos[3 * o + 2] = src[2 * Npad + s];
+}
+// The same to pinned host memory, elements first .. first + count of the
+// caller's vector, or a copy of src where iperm is null; then posts seq, when
+// the grid is small enough to do so itself (Post).  Bound by the link, which
+// takes 53 GB/s.
+constexpr int PUSH = 4;   // elements per thread
+__global__ void __launch_bounds__(BLOCK)
+k_push(double* __restrict__ host, const double* __restrict__ src, const int* __restrict__ iperm, size_t first,
+       size_t count, int Npad, unsigned long long* __restrict__ hostSeq, unsigned long long seq,
+       unsigned int* __restrict__ ticket) {
+#pragma unroll
+  for (int u = 0; u < PUSH; u++) {
+    const size_t x = ((size_t)blockIdx.x * PUSH + u) * BLOCK + threadIdx.x, e = first + x;
+    if (x >= count) break;
+    const size_t atom = e / 3;
+    host[x] = iperm ? src[(e - 3 * atom) * Npad + iperm[atom]] : src[e];
+  }
+  if (!ticket) return;
+  __threadfence_system();
+  __syncthreads();
+  if (last_block(ticket, gridDim.x) && threadIdx.x == 0) {
+    __threadfence_system();
+    *(volatile unsigned long long*)hostSeq = seq;
+  }
+}
+__global__ void k_post_seq(unsigned long long* hostSeq, unsigned long long seq) {
+  __threadfence_system();
+  *(volatile unsigned long long*)hostSeq = seq;
 }
 __global__ void k_add_aos(double* __restrict__ dst, const double* __restrict__ aos,
                           const int* __restrict__ perm, int N, int Npad) {
@@ -2012,7 +2041,8 @@ Device* dev_create(const DeviceSetup& s) {
   d->tmpP.alloc(3 * (size_t)Np); d->tmpQ.alloc(Np);
   d->tmpBody.alloc(Np); d->tmpPerm.alloc(Np); d->tmpFree.alloc(Np); d->tmpCharged.alloc(Np);
   d->stage.alloc(3 * (size_t)std::max(s.N, 1));
-  HIP_CHECK(hipHostMalloc(&d->hstage, 3 * sizeof(double) * std::max(s.N, 1), hipHostMallocDefault));
+  HIP_CHECK(hipHostMalloc((void**)&d->hstage, 3 * sizeof(double) * std::max(s.N, 1), hipHostMallocCoherent));
+  HIP_CHECK(hipHostGetDevicePointer((void**)&d->hstageDev, d->hstage, 0));
   HIP_CHECK(hipHostMalloc(&d->hresult, 64 * sizeof(double), hipHostMallocDefault));
   HIP_CHECK(hipHostMalloc((void**)&d->hpost, 64 * sizeof(double), hipHostMallocCoherent));
   HIP_CHECK(hipHostMalloc((void**)&d->hseq, 64, hipHostMallocCoherent));
@@ -2170,36 +2200,43 @@ static void upload_aos(Device* d, double* dst, const double* host, const int* ma
   launch_check("gather_aos");
   HIP_CHECK(hipStreamSynchronize(d->stream));
 }
-static void download_aos(Device* d, double* host, const double* src) {
-  int N = d->N;
-  hipLaunchKernelGGL(k_scatter_aos, dim3(div_up(N, BLOCK)), dim3(BLOCK), 0, d->stream, d->stage.p, src, d->perm.p, N, d->Npad);
-  launch_check("scatter_aos");
-  HIP_CHECK(hipMemcpyAsync(d->hstage, d->stage.p, 3 * sizeof(double) * N, hipMemcpyDeviceToHost, d->stream));
-  HIP_CHECK(hipStreamSynchronize(d->stream));
-  memcpy(host, d->hstage, 3 * sizeof(double) * N);
+// n doubles to the host: atom by atom from the components of src (iperm
+// given), or as they lie in src.
+static void download(Device* d, double* host, const double* src, const int* iperm) {
+  const size_t n = 3 * (size_t)d->N;
+  const unsigned long long seq0 = d->seq + 1;
+  const ReadRing ring{ d->hstage, d->hstageDev, d->hseq, n };
+  read_back(host, n, ring, seq0, [&](size_t first, size_t count, double* to, unsigned long long seq) {
+    const int g = div_up((long)count, PUSH * BLOCK);
+    unsigned int* ticket = g <= FINISH_BLOCKS ? d->tickets + TICKET_PUSH : nullptr;
+    hipLaunchKernelGGL(k_push, dim3(g), dim3(BLOCK), 0, d->stream, to, src, iperm, first, count, d->Npad, d->hseqDev, seq,
+                       ticket);
+    if (!ticket) hipLaunchKernelGGL(k_post_seq, dim3(1), dim3(1), 0, d->stream, d->hseqDev, seq);
+    launch_check("download");
+    d->seq = seq;
+  }, [&](unsigned long long seq) { post_wait(d, seq); });
 }
 
 void dev_upload_positions(Device* d, const double* R) {
   d->posWrites++;
   if (d->N) upload_aos(d, d->R.p, R, nullptr);
 }
-void dev_download_positions(Device* d, double* R) { if (d->N) download_aos(d, R, d->R.p); }
+void dev_download_positions(Device* d, double* R) { if (d->N) download(d, R, d->R.p, d->iperm.p); }
 void dev_upload_momenta(Device* d, const double* P) { if (d->N) upload_aos(d, d->P.p, P, d->freeFlag.p); }
 void dev_download_momenta(Device* d, double* P) {
   int N = d->N;
   if (!N) return;
+  if (d->bodies.nb == 0) return download(d, P, d->P.p, d->iperm.p);
   hipLaunchKernelGGL(k_scatter_aos, dim3(div_up(N, BLOCK)), dim3(BLOCK), 0, d->stream, d->stage.p, d->P.p, d->perm.p, N, d->Npad);
   launch_check("scatter_aos");
   dev_bodies_particle_momenta(d);
-  HIP_CHECK(hipMemcpyAsync(d->hstage, d->stage.p, 3 * sizeof(double) * N, hipMemcpyDeviceToHost, d->stream));
-  HIP_CHECK(hipStreamSynchronize(d->stream));
-  memcpy(P, d->hstage, 3 * sizeof(double) * N);
+  download(d, P, d->stage.p, nullptr);
 }
 void dev_upload_forces(Device* d, int layer, const double* F) {
   if (d->N) upload_aos(d, d->F.p + 3 * (size_t)d->Npad * layer, F, nullptr);
 }
 void dev_download_forces(Device* d, int layer, double* F) {
-  if (d->N) download_aos(d, F, d->F.p + 3 * (size_t)d->Npad * layer);
+  if (d->N) download(d, F, d->F.p + 3 * (size_t)d->Npad * layer, d->iperm.p);
 }
 void dev_add_forces(Device* d, int layer, const double* F) {
   int N = d->N;

@@ -201,7 +201,7 @@ __device__ __forceinline__ void finish_sums(const Post& post, double* __restrict
 constexpr int POST_PAIRS = 8, POST_EWALD = 16, POST_MODEL = 24, POST_BODY_KE = 32, POST_BODY_W = 40, POST_LOWK = 48,
               POST_TRIG = 56, POST_LIST = 60;
 // Tickets of the kernels that finish their own sums
-enum { TICKET_KE, TICKET_TRIG, TICKET_BODY_KE, TICKET_BODY_W, TICKETS };
+enum { TICKET_KE, TICKET_TRIG, TICKET_BODY_KE, TICKET_BODY_W, TICKET_PUSH, TICKETS };
 
 template <typename T>
 struct DBuf {
@@ -245,7 +245,8 @@ struct Device {
   DBuf<int> tmpI, tmpBody, tmpPerm, tmpFree, tmpCharged;
   // transfers
   DBuf<double> stage;     // 3N AoS, original order
-  double* hstage = nullptr;  // pinned host mirror
+  double* hstage = nullptr;  // pinned host mirror, and its device address
+  double* hstageDev = nullptr;
   // cells
   int M = 0, ncells = 0;
   DBuf<int> key, cellCount, cellStart, order, blockSums;   // cellStart has ncells+1 entries

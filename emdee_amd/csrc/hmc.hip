@@ -33,6 +33,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -43,6 +44,7 @@
 
 #include "../../include/emdee_gpu.h"
 #include "device_state.h"
+#include "readback.h"
 
 namespace emdee {
 
@@ -521,10 +523,16 @@ k_hmc(const ReplicaDesc* __restrict__ desc, const int* __restrict__ order, HmcSt
 }
 
 // Coordinates of every replica as a host takes them, three values per atom.
-__global__ void k_hmc_coords(double* __restrict__ out, const double* __restrict__ R, size_t total) {
-  const size_t i = (size_t)blockIdx.x * BLOCK + threadIdx.x;
-  if (i < total)
-    for (int c = 0; c < 3; c++) out[3 * i + c] = R[c * total + i];
+// elements first .. first + count of the coordinates, atom by atom, to pinned
+// host memory
+__global__ void __launch_bounds__(BLOCK)
+k_hmc_coords(double* __restrict__ host, const double* __restrict__ R, size_t total, size_t first, size_t count) {
+  const size_t x = (size_t)blockIdx.x * BLOCK + threadIdx.x, e = first + x, atom = e / 3;
+  if (x < count) host[x] = R[(e - 3 * atom) * total + atom];
+}
+__global__ void k_hmc_post(unsigned long long* hostSeq, unsigned long long seq) {
+  __threadfence_system();
+  *(volatile unsigned long long*)hostSeq = seq;
 }
 
 }  // namespace emdee
@@ -543,7 +551,11 @@ struct EmDeeHMC {
   DBuf<ReplicaDesc> desc;
   DBuf<int> order, cycle;
   DBuf<double> R, P, F, Rsave, Fsave;   // [3][total]
-  DBuf<double> coords;                  // [total][3], for EmDeeHMC_get
+  // pinned coherent host memory that EmDeeHMC_get reads through: HMC_RING
+  // doubles and the number of the last chunk posted
+  double* ring = nullptr;
+  double* ringDev = nullptr;
+  unsigned long long posted = 0;
   DBuf<double> U, lastDH;
   DBuf<long long> accepted;
   int cap = 0;                   // Verlet-list entries per atom
@@ -570,6 +582,7 @@ const Variant VARIANTS[] = {
   { 1024, 2, k_hmc<1024, 2, true>, k_hmc<1024, 2, false> },
 };
 constexpr int NVARIANTS = 6;
+constexpr size_t HMC_RING = 4 * READ_CHUNK;   // 8 MB
 
 bool variant_fits(const EmDeeHMC* h, int v) {
   for (const ReplicaDesc& d : h->hdesc) {
@@ -651,6 +664,9 @@ EmDeeHMC* EmDeeHMC_create(int nrep, const int* natoms, const double* box, const 
   for (DBuf<double>* b : { &h->R, &h->P, &h->F, &h->Rsave, &h->Fsave }) b->alloc(3 * (size_t)off);
   h->nlist.alloc((size_t)off * h->cap); h->nnb.alloc(off); h->qbuild.alloc(off); h->lstate.alloc(nrep);
   h->Uhist.alloc((size_t)HMC_HIST * nrep);
+  HIP_CHECK(hipHostMalloc((void**)&h->ring, sizeof(double) * (HMC_RING + 8), hipHostMallocCoherent));
+  HIP_CHECK(hipHostGetDevicePointer((void**)&h->ringDev, h->ring, 0));
+  *reinterpret_cast<unsigned long long*>(h->ring + HMC_RING) = 0;
   std::vector<double> Rc(3 * (size_t)off);
   for (int i = 0; i < off; i++) for (int c = 0; c < 3; c++) Rc[(size_t)c * off + i] = R[3 * (size_t)i + c];
   HIP_CHECK(hipMemcpy(h->R.p, Rc.data(), sizeof(double) * Rc.size(), hipMemcpyHostToDevice));
@@ -741,12 +757,22 @@ void EmDeeHMC_synchronize(EmDeeHMC* h) { HIP_CHECK(hipStreamSynchronize(h->strea
 void EmDeeHMC_get(EmDeeHMC* h, double* R, double* U, long long* accepted, double* lastDH) {
   HIP_CHECK(hipStreamSynchronize(h->stream));
   if (R) {
-    h->coords.alloc(3 * (size_t)h->total);
-    hipLaunchKernelGGL(k_hmc_coords, dim3(div_up(h->total, BLOCK)), dim3(BLOCK), 0, h->stream, h->coords.p, h->R.p,
-                       (size_t)h->total);
-    launch_check("hmc coordinates");
-    HIP_CHECK(hipMemcpyAsync(R, h->coords.p, 3 * sizeof(double) * h->total, hipMemcpyDeviceToHost, h->stream));
-    HIP_CHECK(hipStreamSynchronize(h->stream));
+    const volatile unsigned long long* seq = reinterpret_cast<unsigned long long*>(h->ring + HMC_RING);
+    const ReadRing ring{ h->ring, h->ringDev, seq, HMC_RING };
+    const size_t T = h->total;
+    read_back(R, 3 * T, ring, h->posted + 1, [&](size_t first, size_t count, double* to, unsigned long long number) {
+      hipLaunchKernelGGL(k_hmc_coords, dim3(div_up((long)count, BLOCK)), dim3(BLOCK), 0, h->stream, to, h->R.p, T, first,
+                         count);
+      hipLaunchKernelGGL(k_hmc_post, dim3(1), dim3(1), 0, h->stream,
+                         reinterpret_cast<unsigned long long*>(h->ringDev + HMC_RING), number);
+      launch_check("hmc coordinates");
+      h->posted = number;
+    }, [&](unsigned long long number) {
+      for (int k = 0; k < (1 << 20) && *seq < number; k++) __builtin_ia32_pause();
+      if (*seq < number) HIP_CHECK(hipStreamSynchronize(h->stream));
+      if (*seq < number) fatal("batched HMC", "the coordinates did not arrive");
+      std::atomic_thread_fence(std::memory_order_acquire);
+    });
   }
   if (U) HIP_CHECK(hipMemcpy(U, h->U.p, sizeof(double) * h->nrep, hipMemcpyDeviceToHost));
   if (accepted) HIP_CHECK(hipMemcpy(accepted, h->accepted.p, sizeof(long long) * h->nrep, hipMemcpyDeviceToHost));
@@ -785,8 +811,9 @@ void EmDeeHMC_destroy(EmDeeHMC* h) {
   if (h->exec) (void)hipGraphExecDestroy(h->exec);
   if (h->graph) (void)hipGraphDestroy(h->graph);
   h->desc.release(); h->order.release(); h->cycle.release(); h->U.release(); h->lastDH.release(); h->accepted.release();
-  for (DBuf<double>* b : { &h->R, &h->P, &h->F, &h->Rsave, &h->Fsave, &h->coords }) b->release();
+  for (DBuf<double>* b : { &h->R, &h->P, &h->F, &h->Rsave, &h->Fsave }) b->release();
   h->nlist.release(); h->nnb.release(); h->qbuild.release(); h->lstate.release(); h->Uhist.release();
+  if (h->ring) (void)hipHostFree(h->ring);
   (void)hipStreamDestroy(h->stream);
   delete h;
 }
