@@ -15,6 +15,7 @@
 
 #include "device_state.h"
 #include "engine.h"
+#include "trigger.h"
 
 namespace emdee {
 
@@ -561,12 +562,15 @@ __device__ __forceinline__ bool rotate_series2(BodyReg& b, double dt, int h) {
 
 // delta_k = Ct(q) (B(q) d_k) for every member; R_k = rcm + delta_k when R given
 __device__ __forceinline__ void place_member(const BodyState& B, int k, int s, const double (&d)[3], const double* Bm,
-                                             const double* Cm, const double* rc, double* R, int Npad) {
+                                             const double* Cm, const double* rc, double* R, int Npad, double (&r)[3]) {
   double t[4], dl[3];
   mul43(Bm, d, t);
   mul34t(Cm, t, dl);
-  for (int x = 0; x < 3; x++) B.delta.p[x * B.nm + k] = dl[x];
-  if (R) for (int x = 0; x < 3; x++) R[x * Npad + s] = rc[x] + dl[x];
+  for (int x = 0; x < 3; x++) {
+    B.delta.p[x * B.nm + k] = dl[x];
+    r[x] = rc[x] + dl[x];
+    if (R) R[x * Npad + s] = r[x];
+  }
 }
 __device__ void place_members(const BodyState& B, int b, const double* q, double* R, const int* iperm, int Npad) {
   double Bm[12], Cm[12];
@@ -575,7 +579,8 @@ __device__ void place_members(const BodyState& B, int b, const double* q, double
   double rc[3] = { B.rcm.p[b], B.rcm.p[nb + b], B.rcm.p[2 * nb + b] };
   for (int k = B.start.p[b]; k < B.start.p[b + 1]; k++) {
     const double d[3] = { B.d.p[k], B.d.p[nm + k], B.d.p[2 * nm + k] };
-    place_member(B, k, R ? iperm[B.orig.p[k]] : 0, d, Bm, Cm, rc, R, Npad);
+    double r[3];
+    place_member(B, k, R ? iperm[B.orig.p[k]] : 0, d, Bm, Cm, rc, R, Npad, r);
   }
 }
 
@@ -717,46 +722,68 @@ __global__ void k_body_boost(BodyState B, const double* __restrict__ F, const in
 // values in registers instead of spilling at the default 1024-thread bound)
 // Two lanes per body (lanes 2b, 2b+1), which share the exact rotation: the
 // power series where it serves the step, else the closed form; lane 0 stores.
-__global__ void __launch_bounds__(BLOCK) k_body_move(BodyState B, double* __restrict__ R, const int* __restrict__ iperm, double CR, double CP,
-                            double dt, int translate, int rotate, int mode, int Npad) {
+// TRIG: every atom is a member and moves here, so that the kernel also forms
+// pass A of the rebuild trigger for the new positions and their scaled copies,
+// as k_displace_u2_trig does for free atoms (without it a kernel that reads
+// them again: r-RESPA block of 3,000 water atoms 1.45 -> 1.41 ms, ten steps of
+// 98,304 3.72 -> 3.70 ms).
+template <bool TRIG>
+__global__ void __launch_bounds__(BLOCK)
+k_body_move(BodyState B, double* __restrict__ R, const int* __restrict__ iperm, double CR, double CP, double dt,
+            int translate, int rotate, int mode, int Npad, const double* __restrict__ R0, Scaled sc,
+            double* __restrict__ part, double* __restrict__ trig, Post post) {
   const int gt = blockIdx.x * blockDim.x + threadIdx.x, b = gt >> 1, h = gt & 1;
-  if (b >= B.nb) return;   // both lanes of a body
-  const int nb = B.nb, nm = B.nm, k0 = B.start.p[b], k1 = B.start.p[b + 1];
-  // both lanes hold the new centre of mass, lane 0 stores it
-  double rc[3];
-  for (int x = 0; x < 3; x++) {
-    rc[x] = B.rcm.p[x * nb + b];
-    if (translate) rc[x] = CR * rc[x] + CP * B.invMass.p[b] * B.pcm.p[x * nb + b];
-  }
-  if (translate && h == 0)
-    for (int x = 0; x < 3; x++) B.rcm.p[x * nb + b] = rc[x];
-  if (rotate) {
-    BodyReg r;
-    load_body(B, b, r);
-    // lane h places members h, h + 2, ...; what the first needs is on its way
-    // while the body turns (4,096 molecules: 13.4 -> 12.7 us)
-    const bool both = mode == 0;
-    const int step = both ? 2 : 1, first = both ? k0 + h : h == 0 ? k0 : k1;
-    int s0 = 0;
-    double d0[3] = { 0, 0, 0 };
-    if (first < k1) {
-      s0 = iperm[B.orig.p[first]];
-      for (int x = 0; x < 3; x++) d0[x] = B.d.p[x * nm + first];
+  double far = -1.0;
+  int farIdx = INT_MAX;
+  if (b < B.nb) {   // both lanes of a body
+    const int nb = B.nb, nm = B.nm, k0 = B.start.p[b], k1 = B.start.p[b + 1];
+    // both lanes hold the new centre of mass, lane 0 stores it
+    double rc[3];
+    for (int x = 0; x < 3; x++) {
+      rc[x] = B.rcm.p[x * nb + b];
+      if (translate) rc[x] = CR * rc[x] + CP * B.invMass.p[b] * B.pcm.p[x * nb + b];
     }
-    if (both) {
-      if (!rotate_series2(r, dt, h)) rotate_exact2(r, dt, h);
-    } else if (h == 0) rotate_no_squish(r, dt, mode);
-    if (h == 0) store_motion(B, b, r);
-    double Bm[12], Cm[12];
-    matB(r.q, Bm); matC(r.q, Cm);
-    for (int k = first; k < k1; k += step) {
-      if (k > first) {
-        s0 = iperm[B.orig.p[k]];
+    if (translate && h == 0)
+      for (int x = 0; x < 3; x++) B.rcm.p[x * nb + b] = rc[x];
+    if (rotate) {
+      BodyReg r;
+      load_body(B, b, r);
+      // lane h places members h, h + 2, ...; what the first needs is on its way
+      // while the body turns (4,096 molecules: 13.4 -> 12.7 us)
+      const bool both = mode == 0;
+      const int step = both ? 2 : 1, first = both ? k0 + h : h == 0 ? k0 : k1;
+      int o = 0, s = 0;
+      double d0[3] = { 0, 0, 0 };
+      auto fetch = [&](int k) {
+        o = B.orig.p[k];
+        s = iperm[o];
         for (int x = 0; x < 3; x++) d0[x] = B.d.p[x * nm + k];
+      };
+      if (first < k1) fetch(first);
+      if (both) {
+        if (!rotate_series2(r, dt, h)) rotate_exact2(r, dt, h);
+      } else if (h == 0) rotate_no_squish(r, dt, mode);
+      if (h == 0) store_motion(B, b, r);
+      double Bm[12], Cm[12];
+      matB(r.q, Bm); matC(r.q, Cm);
+      for (int k = first; k < k1; k += step) {
+        if (k > first) fetch(k);
+        double rn[3];
+        place_member(B, k, s, d0, Bm, Cm, rc, R, Npad, rn);
+        if (TRIG) {
+          double v;
+          {
+#pragma clang fp contract(off)
+            double dx = rn[0] - R0[s], dy = rn[1] - R0[Npad + s], dz = rn[2] - R0[2 * Npad + s];
+            v = dx * dx + dy * dy + dz * dz;
+          }
+          if (v > far || (v == far && o < farIdx)) { far = v; farIdx = o; }
+          scale_vals(sc, rn[0], rn[1], rn[2], s);
+        }
       }
-      place_member(B, k, s0, d0, Bm, Cm, rc, R, Npad);
     }
   }
+  if (TRIG) trig_block(post, trig, part, far, farIdx);
 }
 
 // rigid_body_virial partials: EmDeeData.f90:926-953
@@ -991,8 +1018,16 @@ void dev_bodies_move(Device* d, double CR, double CP, double dt, bool translate,
   d->posWrites++;
   BodyState& B = d->bodies;
   if (B.nb == 0) return;
-  hipLaunchKernelGGL(k_body_move, dim3(div_up(2L * B.nb, BLOCK)), dim3(BLOCK), 0, d->stream, B, d->R.p, d->iperm.p, CR, CP, dt,
-                     (int)translate, (int)rotate, mode, d->Npad);
+  const int g = div_up(2L * B.nb, BLOCK);
+  if (translate && rotate && d->nfree == 0 && d->trigKnown && g <= d->Npad / BLOCK + 1) {
+    const Post post = dev_post(d, POST_TRIG, TICKET_TRIG, g, false);
+    hipLaunchKernelGGL(k_body_move<true>, dim3(g), dim3(BLOCK), 0, d->stream, B, d->R.p, d->iperm.p, CR, CP, dt, 1, 1, mode,
+                       d->Npad, d->R0.p, dev_trig_scaled(d), d->trigPart.p, d->trig.p, post);
+    dev_trig_formed(d, post, g);
+  } else {
+    hipLaunchKernelGGL(k_body_move<false>, dim3(g), dim3(BLOCK), 0, d->stream, B, d->R.p, d->iperm.p, CR, CP, dt,
+                       (int)translate, (int)rotate, mode, d->Npad, nullptr, Scaled{}, nullptr, nullptr, Post{});
+  }
   launch_check("body move");
 }
 
