@@ -222,10 +222,12 @@ __global__ void __launch_bounds__(1024) k_sg_rows(int* __restrict__ rowSlot, int
 }
 
 // Single-precision positions and species for the gathers of the descriptor
-// kernel: one 16-byte load per neighbour.
+// kernel: one 16-byte load per neighbour.  Clears that kernel's overflow flag
+// (a fill of its own took 4.6 us: proposal of ten steps 2.70 -> 2.68 ms).
 __global__ void k_sg_pos(float4* __restrict__ Rf, const double* __restrict__ R, const int* __restrict__ type, int N,
-                         int Npad) {
+                         int Npad, int* __restrict__ over) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) *over = 0;
   if (i < N) Rf[i] = make_float4((float)R[i], (float)R[Npad + i], (float)R[2 * Npad + i], __int_as_float(type[i]));
 }
 
@@ -927,9 +929,8 @@ static void launch_desc(EmDeeSurrogate* s, Device* d, const SurrogateContext& c,
     s->nearOver.alloc(1);
     s->nearRows = Np;
   }
-  HIP_CHECK(hipMemsetAsync(s->nearOver.p, 0, sizeof(int), d->stream));
   hipLaunchKernelGGL(k_sg_pos, dim3(div_up(d->N, BLOCK)), dim3(BLOCK), 0, d->stream, s->Rf.p, d->R.p, d->type.p, d->N,
-                     Np);
+                     Np, s->nearOver.p);
   int g = div_up(d->N, BLOCK / 64);
   const float* m = normalised ? s->xmean.p : nullptr;
   const float* sd = normalised ? s->xstd.p : nullptr;
