@@ -2534,12 +2534,10 @@ void dev_compute_pairs(Device* d, const PairCall& c, ForceSums* out) {
   launch_check("pairs");
   // the pair sums have a slot of their own, so that a later post (the
   // kinetic energy of the kick that follows a deferred call) leaves them; in
-  // a deferred call they wait for a small kernel that finishes its own sums
-  // (the kick of the free atoms or the body virial) and takes them along
+  // a deferred call they wait for the sums of a later kernel (the kick of the
+  // free atoms or the body virial), which take them along
   d->pairPending = gp;
-  const bool small = d->bodies.nb > 0 ? d->bodies.nb <= FINISH_BLOCKS * BLOCK
-                                      : N <= (d->uniformFree ? 2 : 1) * FINISH_BLOCKS * BLOCK;
-  if (!c.defer || !small) dev_flush_pairs(d);
+  if (!c.defer) dev_flush_pairs(d);
   launch_check("reduce");
   if (!c.defer) dev_pairs_result(d, out);
 }

@@ -190,6 +190,32 @@ __device__ __forceinline__ void finish_sums(const Post& post, double* __restrict
     *(volatile unsigned long long*)post.hostSeq = post.seq;
   }
 }
+// k_reduce_post for sums that a larger grid left in part, and beside it, in a
+// second block, the pair sums that wait: they cost no launch of their own
+// (150,001 LJ atoms, 20 steps 1.89 -> 1.85 ms; 1,048,576 6.56 -> 6.50).  The block with the last ticket posts.
+template <int NV>
+__global__ void k_reduce_post_pairs(Post post, const double* __restrict__ part, int nb, unsigned int* __restrict__ ticket) {
+  if (blockIdx.x == 0) {
+    double v[NV];
+    sum_partials<NV>(v, part, nb);
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int k = 0; k < NV; k++) post.host[k] = v[k];
+    }
+  } else {
+    double w[4];
+    sum_partials<4>(w, post.pairPart, post.pairN);
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) post.pairHost[k] = w[k];
+    }
+  }
+  if (threadIdx.x == 0) __threadfence_system();
+  if (last_block(ticket, 2) && threadIdx.x == 0) {
+    __threadfence_system();
+    *(volatile unsigned long long*)post.hostSeq = post.seq;
+  }
+}
 
 // ------------------------------------------------------------ device state
 
@@ -201,7 +227,7 @@ __device__ __forceinline__ void finish_sums(const Post& post, double* __restrict
 constexpr int POST_PAIRS = 8, POST_EWALD = 16, POST_MODEL = 24, POST_BODY_KE = 32, POST_BODY_W = 40, POST_LOWK = 48,
               POST_TRIG = 56, POST_LIST = 60;
 // Tickets of the kernels that finish their own sums
-enum { TICKET_KE, TICKET_TRIG, TICKET_BODY_KE, TICKET_BODY_W, TICKET_PUSH, TICKETS };
+enum { TICKET_KE, TICKET_TRIG, TICKET_BODY_KE, TICKET_BODY_W, TICKET_PUSH, TICKET_PAIRS, TICKETS };
 
 template <typename T>
 struct DBuf {
@@ -335,8 +361,7 @@ void launch_check(const char* what);
 // finish_sums).
 inline Post dev_post(Device* d, int slot, int ticket, int blocks, bool sums = true) {
   Post p{ d->hpostDev + slot, d->hseqDev, ++d->seq, nullptr, nullptr, nullptr, 0 };
-  if (blocks > FINISH_BLOCKS) return p;
-  p.ticket = d->tickets + ticket;
+  if (blocks <= FINISH_BLOCKS) p.ticket = d->tickets + ticket;
   if (sums && d->pairPending) {
     p.pairPart = d->pairPart;
     p.pairHost = d->hpostDev + POST_PAIRS;
@@ -349,7 +374,11 @@ inline Post dev_post(Device* d, int slot, int ticket, int blocks, bool sums = tr
 // ... whose reduction is launched here when the kernel does not finish it
 template <int NV>
 inline void dev_post_reduce(Device* d, const Post& post, const double* part, int blocks) {
-  if (!post.ticket)
+  if (post.ticket) return;
+  if (post.pairN)
+    hipLaunchKernelGGL(k_reduce_post_pairs<NV>, dim3(2), dim3(BLOCK), 0, d->stream, post, part, blocks,
+                       d->tickets + TICKET_PAIRS);
+  else
     hipLaunchKernelGGL(k_reduce_post<NV>, dim3(1), dim3(BLOCK), 0, d->stream, post.host, post.hostSeq, post.seq, part, blocks);
 }
 // Pair sums that no later kernel took along are reduced and posted now.
