@@ -95,10 +95,8 @@ __global__ void k_reduce_partials(double* __restrict__ out, const double* __rest
 // coherent host memory followed by a sequence number: the host polls the
 // number (post_wait) instead of copying the totals back and waiting on the
 // stream, which saves a copy launch and the wake-up latency of a stream wait
-// on every energy, kinetic-energy and list-trigger read.  (Finishing the
-// reduction in the last block of the producing kernel instead would need a
-// device-scope release fence per block, which writes back the XCD's L2 and
-// costs more than the launch it saves.)
+// on every energy, kinetic-energy and list-trigger read.  (Small grids finish
+// the reduction in the producing kernel: finish_sums.)
 template <int NV>
 __global__ void k_reduce_post(double* __restrict__ host, unsigned long long* __restrict__ hostSeq,
                               unsigned long long seq, const double* __restrict__ partials, int nblocks) {
