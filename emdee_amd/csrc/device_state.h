@@ -367,10 +367,13 @@ void launch_check(const char* what);
 // Where a kernel of `blocks` blocks posts its totals, under the next sequence
 // number; no ticket when the grid is too large to finish them itself.  Pair
 // sums that wait for their reduction go along (sums: the kernel ends in
-// finish_sums).
+// finish_sums, and dev_post_reduce follows).  Every number taken is posted, so
+// that d->seq can be waited for: a trigger's pass A (not sums) on a large grid
+// posts nothing and takes none.
 inline Post dev_post(Device* d, int slot, int ticket, int blocks, bool sums = true) {
-  Post p{ d->hpostDev + slot, d->hseqDev, ++d->seq, nullptr, nullptr, nullptr, 0 };
+  Post p{ d->hpostDev + slot, d->hseqDev, 0, nullptr, nullptr, nullptr, 0 };
   if (blocks <= FINISH_BLOCKS) p.ticket = d->tickets + ticket;
+  if (sums || p.ticket) p.seq = ++d->seq;
   if (sums && d->pairPending) {
     p.pairPart = d->pairPart;
     p.pairHost = d->hpostDev + POST_PAIRS;
