@@ -34,6 +34,7 @@
 
 #include "device_state.h"
 #include "engine.h"
+#include "lanes.h"
 #include "pair_eval.h"
 #include "readback.h"
 #include "trigger.h"
@@ -2468,24 +2469,7 @@ void dev_compute_pairs(Device* d, const PairCall& c, ForceSums* out) {
   hipEvent_t e0 = d->profiling ? d->ev0 : nullptr, e1 = d->profiling ? d->ev1 : nullptr;
   bool U = c.ntypes == 1;
   bool LJ = lj_path(d, c.layer);
-  // threads per atom, 1, 4, 16, 32 or 64: enough wavefronts to fill the chip (at least 2^18
-  // lanes) and about 24 list entries per lane, so that long lists (water at
-  // rc 10 A holds ~700 entries per atom) are spread over many waves
-  int tpa = 1;
-  if (!LJ) {
-    long lanes = std::max(1L << 18, (long)(d->listEntries / 24.0));
-    long want = lanes / std::max(N, 1);
-    tpa = want >= 16 ? 16 : (want >= 4 ? 4 : 1);
-    // small systems with long lists go further, where 16 lanes leave SIMDs
-    // without a wave: a wave per atom up to 4,096 atoms with at least 96
-    // entries (3,000 water atoms, 726 entries: 40 -> 23 us; 800 LJ atoms, 120
-    // entries: step 52 -> 49 us; 4,000 LJ atoms with 75 entries: 60 -> 63 us,
-    // so they keep 16), 32 lanes up to 16,384 atoms with at least 384
-    // (12,288 water atoms: step 315 -> 311 us; 98,304: 598 -> 612 us)
-    const double each = d->listEntries / std::max(N, 1);
-    if (N <= 4096 && want >= 64 && each >= 96.0) tpa = 64;
-    else if (N <= 16384 && want >= 24 && each >= 384.0) tpa = 32;
-  }
+  const int tpa = LJ ? 1 : pair_lanes(N, d->listEntries, c.mixed != 0, U);
   int gp = div_up((long)N * tpa, BLOCK);
   // the pair kernels write four sums per block into pairPart, which holds
   // 64 (Npad / BLOCK + 1) values: enough for up to 16 lanes per atom (256

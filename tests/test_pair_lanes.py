@@ -1,0 +1,33 @@
+"""The pair kernels' lanes per atom against measured step times (us) of 16, 32 and 64 lanes: wherever the rule leaves
+16 lanes, that does not cost more than the timings scatter (2 %)."""
+import host_cpp
+
+# atoms, list entries per atom, mixed form, one type, step times of 16, 32 and 64 lanes
+MEASURED = [
+    (800, 120, 0, 1, 42.1, 41.4, 42.1), (1000, 224, 0, 1, 45.0, 43.4, 42.6), (2000, 134, 0, 1, 43.3, 42.4, 43.0),
+    (2000, 320, 0, 1, 48.7, 45.9, 45.0), (2500, 114, 0, 1, 44.3, 44.0, 45.1), (3072, 122, 0, 1, 44.6, 44.4, 45.8),
+    (3072, 349, 0, 1, 51.0, 48.6, 48.3), (3500, 112, 0, 1, 44.5, 44.5, 47.0), (4096, 123, 0, 1, 44.9, 44.4, 47.2),
+    (4096, 155, 0, 1, 46.2, 45.6, 47.2), (4096, 784, 0, 1, 60.8, 54.9, 55.4), (3500, 112, 1, 1, 44.1, 43.0, 45.4),
+    (4096, 155, 1, 1, 43.8, 43.2, 45.2), (3000, 698, 0, 0, 114.5, 107.1, 101.6), (4095, 743, 0, 0, 121.1, 113.3, 110.5),
+    (8192, 727, 0, 1, 67.8, 62.5, 67.4), (10000, 518, 0, 1, 63.4, 67.2, 66.1), (12288, 735, 0, 1, 77.3, 82.4, 82.7),
+    (16384, 704, 0, 1, 80.4, 83.1, 90.5), (8192, 727, 1, 1, 72.9, 62.9, 67.5), (10000, 733, 1, 1, 76.7, 69.7, 73.1),
+    (12288, 735, 1, 1, 79.9, 83.8, 80.6), (12288, 610, 1, 1, 70.7, 73.7, 70.8), (9999, 721, 1, 0, 127.5, 118.6, 121.7),
+    (12288, 601, 1, 0, 124.2, 126.8, 128.2), (9999, 721, 0, 0, 141.8, 135.9, 137.1), (12288, 721, 0, 0, 143.1, 141.8, 144.8),
+]
+
+
+def test_rule_against_measurements(tmp_path):
+    body = "\n".join(f'printf("%d\\n", pair_lanes({n}, {n * e}.0, {m}, {u}));' for n, e, m, u, *_ in MEASURED)
+    chosen = [int(line) for line in host_cpp.run(tmp_path, body, headers=("lanes.h",))]
+    assert len(chosen) == len(MEASURED)
+    for row, lanes in zip(MEASURED, chosen):
+        t = dict(zip((16, 32, 64), row[4:]))
+        assert t[lanes] <= 1.02 * t[16], (row, lanes)
+
+
+def test_rule_at_its_ends(tmp_path):
+    # long lists of large systems, short lists, no atoms and no entries: 16, 4 or 1 lanes as the entries ask
+    args = [(98304, 98304 * 726, 0, 0), (98304, 98304 * 726, 1, 0), (98304, 98304 * 77, 0, 1), (60000, 60000 * 77, 0, 1), (4000, 4000 * 75, 0, 1),
+            (600, 0, 0, 1), (0, 0, 0, 1), (400000, 400000 * 20, 0, 1), (16385, 16385 * 900, 0, 0)]
+    body = "\n".join(f'printf("%d\\n", pair_lanes({n}, {e}.0, {m}, {u}));' for n, e, m, u in args)
+    assert [int(line) for line in host_cpp.run(tmp_path, body, headers=("lanes.h",))] == [16, 16, 1, 4, 16, 16, 16, 1, 16]
