@@ -54,10 +54,12 @@ constexpr int HMC_CMAX = 6144;   // cells per replica
 constexpr int HMC_HIST = 1024;   // cycles of potential-energy history
 const double TWO_PI_D = 6.283185307179586;
 
+// (padded to whole 16-byte groups, as it is loaded: without the pads the plain
+// form's spills fall differently and 512 replicas take 9.4 ms a cycle for 8.8)
 struct ReplicaDesc {
-  int off, N, M, Ml;       // atom offset and count; cells per edge for the force walk and for the list build
+  int off, N, pad0, M;     // atom offset and count; cells per edge for the list build
   double L, kT;
-  float K, lo, hi, fpad;   // fixed-point cutoff band (mixed form)
+  float K, lo, hi, pad1;   // fixed-point cutoff band (mixed form)
   double Rc2s, unit;       // FP64 scaled cutoff; L / 2^32
   double Rl2s, trig2s;     // list radius (rc + skin)^2 and (skin/2)^2, scaled units^2
 };
@@ -285,7 +287,7 @@ k_hmc(const ReplicaDesc* __restrict__ desc, const int* __restrict__ order, HmcSt
   // 3.82; atoms taken in cell order, whose lanes read the same candidates but
   // store apart, 4.35; candidates read four at a time 4.48.
   auto build_list = [&]() {
-    build_cells(d.Ml);
+    build_cells(d.M);
     const float rl2 = (float)(d.Rl2s * 18446744073709551616.0 * (1.0 + 1e-4));
     int over = 0;
     for (int i = threadIdx.x; i < N; i += BS) {
@@ -301,7 +303,7 @@ k_hmc(const ReplicaDesc* __restrict__ desc, const int* __restrict__ order, HmcSt
           *reinterpret_cast<uint2*>(li + 8 * (size_t)(n >> 3) * N + (n & 4)) = make_uint2(lo, hi);
         n++;
       };
-      walk(i, d.Ml, d.Rl2s, [&](int a, int b) __attribute__((always_inline)) {
+      walk(i, d.M, d.Rl2s, [&](int a, int b) __attribute__((always_inline)) {
         for (int q = a; q < b; q++) {
           const int j = s.clist[q];
           const uint2 v = s.qxy[j];
@@ -593,21 +595,22 @@ const Variant VARIANTS[] = {
 constexpr int NVARIANTS = 6;
 constexpr size_t HMC_RING = 4 * READ_CHUNK;   // 8 MB
 
+// cells per edge: of side at least (rc + skin) / div, or one cell
+double edge_cells(const EmDeeHMC* h, const ReplicaDesc& d, int div) {
+  const double M = std::floor(div * d.L / (h->rc + HMC_SKIN));
+  return M >= 2 * div + 1 ? M : 1.0;
+}
+
 bool variant_fits(const EmDeeHMC* h, int v) {
   for (const ReplicaDesc& d : h->hdesc) {
-    int M = std::max(1, (int)std::floor(VARIANTS[v].div * d.L / h->rc));
-    if ((long)M * M * M > HMC_CMAX) return false;
+    const double M = edge_cells(h, d, VARIANTS[v].div);
+    if (M * M * M > HMC_CMAX) return false;
   }
   return true;
 }
 
 void set_cells(EmDeeHMC* h, int div) {
-  for (ReplicaDesc& d : h->hdesc) {
-    int M = std::max(1, (int)std::floor(div * d.L / h->rc));
-    d.M = M >= 2 * div + 1 ? M : 1;
-    int Ml = std::max(1, (int)std::floor(div * d.L / (h->rc + HMC_SKIN)));
-    d.Ml = Ml >= 2 * div + 1 ? Ml : 1;
-  }
+  for (ReplicaDesc& d : h->hdesc) d.M = (int)edge_cells(h, d, div);
   HIP_CHECK(hipMemcpy(h->desc.p, h->hdesc.data(), sizeof(ReplicaDesc) * h->nrep, hipMemcpyHostToDevice));
 }
 
@@ -639,7 +642,7 @@ EmDeeHMC* EmDeeHMC_create(int nrep, const int* natoms, const double* box, const 
     if (natoms[r] < 2 || natoms[r] > HMC_NMAX) fatal(task, "replica sizes must be between 2 and 8192 atoms");
     if (box[r] < 2.0 * rc) fatal(task, "replica box shorter than twice the cutoff");
     ReplicaDesc& d = h->hdesc[r];
-    d.off = off; d.N = natoms[r]; d.M = 1; d.L = box[r]; d.kT = kT[r];
+    d.off = off; d.N = natoms[r]; d.L = box[r]; d.kT = kT[r];
     double two32 = 4294967296.0, rc2s = (rc * rc) / (box[r] * box[r]), rc2u = rc2s * two32 * two32;
     d.K = (float)(two32 * two32 / (box[r] * box[r]));
     // FP32 rounding plus the quantisation of the fixed-point coordinates
