@@ -342,7 +342,6 @@ static bool forces_begin(tEmDee* md, bool defer, ForceSums& fs) {
   c.L = me->L;
   c.invL2 = 1.0 / (me->L * me->L);
   c.Rc2 = (me->useInRc[l] ? me->InRcSq : me->RcSq) * c.invL2;
-  c.scaled = 1;
   fs = ForceSums{ 0, 0, 0, 0 };
   bool pairsOnly = me->nbonds + me->nangles + me->ndihedrals == 0 && !me->coul[l - 1].requires_kspace &&
                    !(me->surrogate && me->surrogateLayer == l) && me->nbodies == 0;

@@ -139,14 +139,6 @@ __global__ void k_gather_scalar(T* __restrict__ dst, const T* __restrict__ src, 
   if (s < N) dst[s] = src[perm[s]];
 }
 
-// Rs = R / L, exactly as EmDeeCode.f90:1228 (IEEE division), packed with
-// the atom type so that a neighbor costs one 32-byte gather.
-__global__ void k_scale4(double4* __restrict__ Rs4, const double* __restrict__ R, const int* __restrict__ type,
-                         double L, int N, int Npad) {
-  int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s < N) Rs4[s] = make_double4(R[s] / L, R[Npad + s] / L, R[2 * Npad + s] / L, (double)type[s]);
-}
-
 // ---- rebuild trigger, neighbor_lists.f90:41-59 ---------------------------
 // With d_k = |R_k - R0_k|^2 in ORIGINAL atom order, the reference returns
 // max + 2 sqrt(max*next) + next where next = d_1 if atom 1 holds the maximum
@@ -227,7 +219,7 @@ __device__ __forceinline__ int cell_coord(double s, int M) {
   int c = (int)(M * (s - floor(s)));
   return c >= M ? c - M : c;
 }
-// Cell of each slot from Rs = R / L (the division of k_scale4), counted per
+// Cell of each slot from Rs = R / L (the division of scale_vals), counted per
 // cell for the counting sort.
 __global__ void k_cell_key(int* __restrict__ key, int* __restrict__ count, const double* __restrict__ R, double L,
                            int M, int N, int Npad) {
@@ -457,22 +449,13 @@ struct MixedCut {
   double L;
 };
 
-__global__ void k_scale4q(double4* __restrict__ Rs4, int4* __restrict__ Q4, float* __restrict__ qf,
-                          const double* __restrict__ R, const int* __restrict__ type, const double* __restrict__ charge,
-                          const int* __restrict__ charged, double L, int N, int Npad) {
-  int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= N) return;
-  Scaled sc{ Rs4, Q4, qf, type, charge, charged, L };
-  scale_slot(sc, R, s, Npad);
-}
-
 // relative half-width of the FP32 band around a cutoff Rc2s (scaled units^2)
 inline double band_rel(double Rc2s) {
   const double q = 1.0 / 4294967296.0;
   return 2e-6 + 4.0 * q / std::sqrt(Rc2s) + 3.0 * q * q / Rc2s;
 }
 
-// The same test from the unscaled positions: Rs = R / L as k_scale4 forms it.
+// The same test from the unscaled positions: Rs = R / L as scale_vals forms it.
 __device__ __noinline__ bool exact_inside_R(const double* __restrict__ R, int Npad, double L, int i, int j,
                                            double Rc2s) {
   double dx = R[i] / L - R[j] / L, dy = R[Npad + i] / L - R[Npad + j] / L, dz = R[2 * Npad + i] / L - R[2 * Npad + j] / L;
@@ -2451,17 +2434,7 @@ void dev_compute_pairs(Device* d, const PairCall& c, ForceSums* out) {
   int N = d->N, Np = d->Npad;
   double* F = d->F.p + 3 * (size_t)Np * c.layer;
   if (N == 0) { *out = ForceSums{ 0, 0, 0, 0 }; return; }
-  int g = div_up(N, BLOCK);
-  if (c.scaled) {
-    // the trigger of this force evaluation (or the list build) wrote them
-  } else if (c.mixed) {
-    d->Q4.alloc(Np);
-    d->qf.alloc(Np);
-    hipLaunchKernelGGL(k_scale4q, dim3(g), dim3(BLOCK), 0, d->stream, d->Rs4.p, d->Q4.p, d->qf.p, d->R.p, d->type.p,
-                       d->charge.p, d->chargedFlag.p, c.L, N, Np);
-  } else {
-    hipLaunchKernelGGL(k_scale4, dim3(g), dim3(BLOCK), 0, d->stream, d->Rs4.p, d->R.p, d->type.p, c.L, N, Np);
-  }
+  // (the scaled positions: written by this evaluation's trigger or list build)
   const DevPair* pt = d->pairs.p + (size_t)c.layer * c.ntypes * c.ntypes;
   const DevCoul* cp = d->couls.p + c.layer;
   // with profiling on, the launch itself records the kernel's start and end

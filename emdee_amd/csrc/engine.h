@@ -81,7 +81,6 @@ struct PairCall {
   int energy;         // Options.Compute
   int mixed;          // FP32 pair arithmetic with FP64 accumulation
   double L, invL2, Rc2;   // box and scaled squared cutoff
-  int scaled;         // scaled positions are current (written by the trigger or the list build)
   int fresh = 0;      // the list was built for these positions
   int defer = 0;      // return once the kernels are queued; dev_pairs_result reads the sums
 };

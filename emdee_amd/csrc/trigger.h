@@ -6,7 +6,7 @@
 namespace emdee {
 
 // Scaled positions of a slot: Rs = R / L (EmDeeCode.f90:1228, IEEE division)
-// with the type, and, when Q4 is given, the mixed form's fixed-point copy
+// packed with the type, so that a neighbour costs one 32-byte gather, and, when Q4 is given, the mixed form's fixed-point copy
 // u = round(2^32 (s - floor s)) mod 2^32 and FP32 charge.
 // Q4.w holds the type; a slot whose scaled position is not finite also
 // carries Q4_NONFINITE, so that the fixed-point prefilter of the list build
