@@ -410,7 +410,7 @@ static void ewald_state_setup(EwaldState* e, const EwaldSetup& s) {
   std::vector<int4> quads;
   std::vector<int> at((size_t)(s.nm + 1) * (s.nm + 1), -1);
   for (int k = 0; k < s.nvecs; k++) {
-    const int n1 = s.kn[4 * k], n2 = std::abs(s.kn[4 * k + 1]), n3 = std::abs(s.kn[4 * k + 2]);
+    const int n1 = s.kn[3 * k], n2 = std::abs(s.kn[3 * k + 1]), n3 = std::abs(s.kn[3 * k + 2]);
     if (n1 < 0 || n1 > s.nm || n2 > s.nm || n3 > s.nm)
       fatal("kspace set-up", "k-vector outside the half space of the table");
     int& q = at[(size_t)n1 * (s.nm + 1) + n2];
@@ -425,9 +425,9 @@ static void ewald_state_setup(EwaldState* e, const EwaldSetup& s) {
   std::vector<double> wq((size_t)e->nq * e->npb * EW_P, 0.0);
   std::vector<int> seen(wq.size(), 0);
   for (int k = 0; k < s.nvecs; k++) {
-    const int n2 = std::abs(s.kn[4 * k + 1]), n3 = std::abs(s.kn[4 * k + 2]);
-    const size_t o = (size_t)at[(size_t)s.kn[4 * k] * (s.nm + 1) + n2] * e->npb * EW_P + n3;
-    wq[o] = s.kv[4 * k + 3];
+    const int n2 = std::abs(s.kn[3 * k + 1]), n3 = std::abs(s.kn[3 * k + 2]);
+    const size_t o = (size_t)at[(size_t)s.kn[3 * k] * (s.nm + 1) + n2] * e->npb * EW_P + n3;
+    wq[o] = s.prefac[k];
     seen[o]++;
   }
   for (size_t q = 0; q < quads.size(); q++)
@@ -501,7 +501,6 @@ static unsigned long long ewald_launch(Device* d, EwaldState* e, double* F, cons
   hipLaunchKernelGGL(k_ew_sigma, dim3(e->nq, e->npb), dim3(512), 0, d->stream, e->D, e->part, e->Mpart, e->quad.p,
                      e->wq.p, vf, e->typeChunks.p, lam, e->nt, e->nq, e->npb);
   launch_check("ewald sigma");
-  const int gk = e->nq * e->npb;
   hipLaunchKernelGGL(k_ew_forces, dim3(e->nslots / (64 * EW_FA), e->ksF), dim3(256), 0, d->stream, e->Fpart, e->T, e->quad.p,
                      e->D, e->groupType.p, e->unit, e->nm, e->nslots, e->nq, e->npb, e->ksF);
   launch_check("ewald forces");

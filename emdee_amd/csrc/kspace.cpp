@@ -151,8 +151,8 @@ EwaldHost ewald_initialize(double accuracy, double Rc, double L, int nlayers, co
   int nvecs = (int)n.size() / 3;
   e.nm = nmax;
   e.nvecs = nvecs;
-  e.kn.resize(4 * (size_t)nvecs);
-  e.kv.resize(4 * (size_t)nvecs);
+  e.kn = n;
+  e.prefac.resize(nvecs);
   double B = -0.25 / (h.alpha * h.alpha);
   h.volume = L * L * L;
   double fourPiByV = 4.0 * PI_ / h.volume;
@@ -160,14 +160,7 @@ EwaldHost ewald_initialize(double accuracy, double Rc, double L, int nlayers, co
     double k[3];
     for (int x = 0; x < 3; x++) k[x] = unit * n[3 * i + x];
     double ksq = k[0] * k[0] + k[1] * k[1] + k[2] * k[2];
-    double prefac = fourPiByV * std::exp(ksq * B) / ksq;
-    for (int x = 0; x < 3; x++) e.kv[4 * i + x] = 2.0 * prefac * k[x];
-    e.kv[4 * i + 3] = prefac;
-    bool cont = i > 0 && n[3 * i] == n[3 * i - 3] && n[3 * i + 1] == n[3 * i - 2] && n[3 * i + 2] == n[3 * i - 1] + 1;
-    e.kn[4 * i] = n[3 * i];
-    e.kn[4 * i + 1] = n[3 * i + 1];
-    e.kn[4 * i + 2] = n[3 * i + 2];
-    e.kn[4 * i + 3] = cont ? 0 : 1;
+    e.prefac[i] = fourPiByV * std::exp(ksq * B) / ksq;
   }
   return h;
 }
@@ -200,21 +193,14 @@ EwaldSetup lowk_setup(const EwaldSetup& full, int layer, double alpha, double L,
   int nvecs = (int)n.size() / 3;
   e.nm = nmax;
   e.nvecs = nvecs;
-  e.kn.assign(4 * (size_t)nvecs, 0);
-  e.kv.assign(4 * (size_t)nvecs, 0.0);
+  e.kn = n;
+  e.prefac.resize(nvecs);
   double B = -0.25 / (alpha * alpha), fourPiByV = 4.0 * PI_ / (L * L * L);
   for (int i = 0; i < nvecs; i++) {
     double k[3];
     for (int x = 0; x < 3; x++) k[x] = unit * n[3 * i + x];
     double ksq = k[0] * k[0] + k[1] * k[1] + k[2] * k[2];
-    double prefac = fourPiByV * std::exp(ksq * B) / ksq;
-    for (int x = 0; x < 3; x++) e.kv[4 * i + x] = 2.0 * prefac * k[x];
-    e.kv[4 * i + 3] = prefac;
-    bool cont = i > 0 && n[3 * i] == n[3 * i - 3] && n[3 * i + 1] == n[3 * i - 2] && n[3 * i + 2] == n[3 * i - 1] + 1;
-    e.kn[4 * i] = n[3 * i];
-    e.kn[4 * i + 1] = n[3 * i + 1];
-    e.kn[4 * i + 2] = n[3 * i + 2];
-    e.kn[4 * i + 3] = cont ? 0 : 1;
+    e.prefac[i] = fourPiByV * std::exp(ksq * B) / ksq;
   }
   return e;
 }

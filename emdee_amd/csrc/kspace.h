@@ -9,9 +9,10 @@
 namespace emdee {
 
 // Everything the k-space kernels need, in the device's order.
-//   * k-vectors in the reference order (kspace_ewald.f90:115-138): n3 runs
-//     fastest, so consecutive vectors that differ only by n3 += 1 form a
-//     "row" along which e^{ik.r} advances by one factor of e^{2 pi i z/L}.
+//   * the k-vectors k = unit n of the half space and their coefficients, in
+//     the reference order (kspace_ewald.f90:115-138), which the device folds
+//     into quads: one (n1, |n2|) with its n3 from 0 to the largest in the
+//     sphere, whose vectors of either sign share products of real tables.
 //   * charged atoms in "slots": grouped by charged type (ascending type,
 //     ascending atom index, modelClass_kspace.f90:130-150), each type padded
 //     with empty slots (item -1, charge 0) to a multiple of EWALD_GROUP so
@@ -22,8 +23,8 @@ struct EwaldSetup {
   int nm = 0, nvecs = 0, nt = 0, nl = 0, nslots = 0;
   double alpha = 0;            // Ewald splitting parameter
   double unit = 0;             // 2 pi / L: k = unit n
-  std::vector<int> kn;         // [nvecs][4]: n1, n2, n3, row-start flag
-  std::vector<double> kv;      // [nvecs][4]: 2 prefac k (x, y, z), prefac
+  std::vector<int> kn;         // [nvecs][3]: n1, n2, n3
+  std::vector<double> prefac;  // [nvecs]: 4 pi / V exp(-k^2 / (4 alpha^2)) / k^2
   std::vector<int> slotItem;   // [nslots]: original atom index (0-based) or -1
   std::vector<double> slotQ;   // [nslots]
   std::vector<int> groupType;  // [nslots / EWALD_GROUP]: local charged type (0-based)
