@@ -125,8 +125,9 @@ struct HmcLds {
 // pass walks an atom's list and gives it both half kicks that its force takes
 // part in (the end of this step and the start of the next), so forces stay in
 // registers except at a trajectory's end; the drift pass moves the atom and
-// renews its fixed-point coordinates.  Per step and atom that is 120 bytes of
-// state instead of 370.  The list holds packets of eight 16-bit entries, one
+// renews its fixed-point coordinates.  Per step and atom that is 136 bytes of
+// state instead of 370 (momenta 72, positions 48, build coordinates 16), and
+// 64 more in the plain form for the scaled positions.  The list holds packets of eight 16-bit entries, one
 // 16-byte load each (four, and the next in flight, instead of eight loads with
 // an address and a bound test apiece), padded with the atom itself, which the
 // pair terms mask.  Bound by instruction issue and the latency of one
@@ -532,9 +533,8 @@ k_hmc(const ReplicaDesc* __restrict__ desc, const int* __restrict__ order, HmcSt
   if (threadIdx.x == 0) lstate[r] = listState;
 }
 
-// Coordinates of every replica as a host takes them, three values per atom.
-// elements first .. first + count of the coordinates, atom by atom, to pinned
-// host memory
+// Elements first .. first + count of all replicas' coordinates, atom by atom,
+// to pinned host memory
 __global__ void __launch_bounds__(BLOCK)
 k_hmc_coords(double* __restrict__ host, const double* __restrict__ R, size_t total, size_t first, size_t count) {
   const size_t x = (size_t)blockIdx.x * BLOCK + threadIdx.x, e = first + x, atom = e / 3;
