@@ -301,10 +301,11 @@ __global__ void k_cell_rank(int* __restrict__ order, const int* __restrict__ sca
 // The whole sort in one workgroup: counts, scan, scatter and ranking in LDS,
 // to the same cellStart and order as the kernels above (a cell's members by
 // ascending original index).  Bound by the chain of its five passes over one
-// CU's LDS, which up to SORT_ATOMS atoms and SORT_CELLS cells costs less than
-// the launches (800 LJ atoms 4.3 us, 4,000 9.2; six kernels and two fills
-// 16 us of their own and 4 us between each).  Larger sorts have more atoms
-// than LDS.
+// CU's LDS, which costs less than the launches of small sorts (800 LJ atoms
+// 4.3 us, 4,000 9.2; six kernels and two fills 16 us of their own and 4 us
+// between each) and no more than those of larger ones, up to the atoms and
+// cells that LDS holds: per list build 8 to 15 us less at 200 to 1,000 atoms, 4
+// to 7 at 2,000 to 6,000, the same within 1 us at 8,000 to 16,384 (rc 2.5).
 constexpr int SORT_ATOMS = 16384, SORT_CELLS = 16384, SORT_T = 1024;
 __global__ void __launch_bounds__(SORT_T)
 k_cell_sort_small(int* __restrict__ order, int* __restrict__ start, const double* __restrict__ R,
@@ -626,7 +627,10 @@ __device__ __forceinline__ void scan_range(int a, int b, int i, double xi, doubl
 // kernels read 486, 560, 640 or 726 of them as the displacement grows, and
 // entries inside the cutoff lie together, so fewer waves run the pair terms
 // for a few lanes only.  12,288 atoms: pair kernel 60 -> 49 us, build 60 -> 69
-// us every ten steps.
+// us every ten steps.  The order alone is worth the build: with the box scaled
+// at every step, when whole lists are read, a step of 98,304 water atoms takes
+// 479 us for 537 without shells, of 12,288 149 for 158 (fixed box: 459 for 523
+// and 142 for 152).
 // The near entries go straight to the list in scan order, the others to LDS
 // until the atom's scan ends and are then sorted by shell; past FAR_CAP they
 // go to the near part, which is always read.  (98,304 atoms: FAR_CAP 160

@@ -115,10 +115,11 @@ __global__ void k_ew_tables(double2* __restrict__ T, const int* __restrict__ ite
 // 256-slot group.  v_mfma_f64_16x16x4: rows i = (quad, e2) with e1 = c in one
 // tile and e1 = s in the other, columns j = n3 with e3 = c and e3 = s in two
 // tiles, four charges per step, so a step's three table loads (X1, X2, X3)
-// feed four products.  Bound by the matrix cores, which reach 42 TF/s in
-// this product of FP64: 12,288 charges, 7,073 vectors took 55 us by complex
-// recursion on the vector units, and take 22 (28 TF/s) here, with two or four
-// wavefronts per block.
+// feed four products.  12,288 charges, 7,073 vectors took 55 us by complex
+// recursion on the vector units, and take 22 (28 TF/s, where a large FP64
+// product reaches 72) here, with two or four wavefronts per block.  Bound by
+// the latency of the table loads and the ends of a short kernel: the matrix
+// cores are busy for 45 % of the time, the waves wait for 74 % of theirs.
 // Mpart[((chunk * nq + quad) * npb + block) * 128 + 64 e1 + 32 e2 + 16 e3 + n3].
 constexpr int EW_SW = 4;                             // wavefronts per block
 __global__ void __launch_bounds__(64 * EW_SW) k_ew_structure(double* __restrict__ Mpart, const double2* __restrict__ T,
@@ -277,9 +278,10 @@ __global__ void __launch_bounds__(512) k_ew_sigma(double* __restrict__ D, double
 // type), so they read the same D.  Per tile of four quads, with rows
 // i = quad + 4 (2 e1 + e2), D times X3 and D times -dX3/d(angle) over the
 // columns give T and T' of 4 x 16 charges: the lane of quad lane/16 and charge
-// lane%16 holds its four (e1, e2) values and finishes with X1 and X2.  Bound
-// by the matrix cores: 12,288 charges, 7,073 vectors: 73 us by recursion, 32
-// here (28 TF/s of products).  EW_FA = 2 tiles of 16 charges per wavefront
+// lane%16 holds its four (e1, e2) values and finishes with X1 and X2.  12,288
+// charges, 7,073 vectors: 73 us by recursion, 32 here (28 TF/s of products),
+// with the matrix cores 41 % busy, VALU issue at 46 % and the waves waiting for
+// 49 % of their cycles.  EW_FA = 2 tiles of 16 charges per wavefront
 // share each load of D at four wavefronts per SIMD; one tile took 34-36 us,
 // four (two wavefronts per SIMD for registers) 35-40.
 __global__ void __launch_bounds__(256) k_ew_forces(double* __restrict__ Fpart, const double2* __restrict__ T,

@@ -127,13 +127,15 @@ struct HmcLds {
 // registers except at a trajectory's end; the drift pass moves the atom and
 // renews its fixed-point coordinates.  Per step and atom that is 136 bytes of
 // state instead of 370 (momenta 72, positions 48, build coordinates 16), and
-// 64 more in the plain form for the scaled positions.  The list holds packets of eight 16-bit entries, one
-// 16-byte load each (four, and the next in flight, instead of eight loads with
-// an address and a bound test apiece), padded with the atom itself, which the
-// pair terms mask.  Bound by instruction issue and the latency of one
-// replica's 16 wavefronts per CU: half the time is the force pass, 45 % the
-// 1.7 list builds of a cycle.  512 replicas of 256 to 8,192 atoms, ten steps:
-// 4.41 -> 3.82 ms a cycle.  Partners read two, four or eight at a time and
+// 64 more in the plain form for the scaled positions.  The list holds packets
+// of eight 16-bit entries, one 16-byte load each (four, and the next in flight,
+// instead of eight loads with an address and a bound test apiece), padded with
+// the atom itself, which the pair terms mask.  Bound by instruction issue (54 %
+// of the chip's, the tail of the launch included) and the latency of one
+// replica's 16 wavefronts per CU: the mixed form spends 46 % of its time in the
+// force passes and 44 % in the 1.7 list builds of a cycle, the plain form 76 and
+// 19 %.  512 replicas of 256 to 8,192 atoms, ten steps: 4.41 -> 3.82 ms a cycle.
+// Partners read two, four or eight at a time and
 // masked instead of branched over: 3.93, 4.11 and 4.04 ms with 1,024 threads,
 // 10 % less with 256, which no replica set of these sizes chooses.
 template <int BS, int DIV, bool MIXED>
