@@ -1,10 +1,11 @@
-"""The pair kernels' lanes per atom against measured step times (us) of 16, 32 and 64 lanes: wherever the rule leaves
-16 lanes, that does not cost more than the timings scatter (2 %)."""
+"""The pair kernels' lanes per atom against measured step times (us) of 16, 32 and 64 lanes: the rule's choice costs no
+more than the timings scatter (1.5 %) over the fastest of the three."""
 import host_cpp
 
 # atoms, list entries per atom, mixed form, one type, step times of 16, 32 and 64 lanes
 MEASURED = [
-    (800, 120, 0, 1, 42.1, 41.4, 42.1), (1000, 224, 0, 1, 45.0, 43.4, 42.6), (2000, 134, 0, 1, 43.3, 42.4, 43.0),
+    (500, 121, 0, 1, 38.16, 37.28, 36.66), (800, 125, 0, 1, 38.90, 37.81, 37.21), (1500, 132, 0, 1, 39.90, 38.59, 38.95),
+    (1000, 224, 0, 1, 45.0, 43.4, 42.6), (2000, 134, 0, 1, 43.3, 42.4, 43.0),
     (2000, 320, 0, 1, 48.7, 45.9, 45.0), (2500, 114, 0, 1, 44.3, 44.0, 45.1), (3072, 122, 0, 1, 44.6, 44.4, 45.8),
     (3072, 349, 0, 1, 51.0, 48.6, 48.3), (3500, 112, 0, 1, 44.5, 44.5, 47.0), (4096, 123, 0, 1, 44.9, 44.4, 47.2),
     (4096, 155, 0, 1, 46.2, 45.6, 47.2), (4096, 784, 0, 1, 60.8, 54.9, 55.4), (3500, 112, 1, 1, 44.1, 43.0, 45.4),
@@ -22,7 +23,7 @@ def test_rule_against_measurements(tmp_path):
     assert len(chosen) == len(MEASURED)
     for row, lanes in zip(MEASURED, chosen):
         t = dict(zip((16, 32, 64), row[4:]))
-        assert t[lanes] <= 1.02 * t[16], (row, lanes)
+        assert t[lanes] <= 1.015 * min(t.values()), (row, lanes)
 
 
 def test_rule_at_its_ends(tmp_path):
