@@ -2032,6 +2032,10 @@ void dev_destroy(Device* d) {
   for (DBuf<int>* b : { &d->type, &d->body, &d->perm, &d->freeFlag, &d->chargedFlag, &d->tmpI, &d->tmpBody, &d->tmpPerm, &d->tmpFree, &d->tmpCharged, &d->key, &d->cellCount, &d->cellStart, &d->order, &d->blockSums, &d->nbr, &d->nnb, &d->flags, &d->exOff, &d->exItem, &d->iperm }) b->release();
   d->pairs.release(); d->couls.release(); d->interact.release(); d->ljt.release(); d->ljk.release(); d->ljt64.release();
   d->ljk64.release();
+  BodyState& B = d->bodies;
+  B.start.release(); B.orig.release();
+  for (DBuf<double>* b : { &B.mMass, &B.d, &B.delta, &B.mass, &B.invMass, &B.MoI, &B.invMoI, &B.coef, &B.rcm, &B.pcm, &B.q,
+                           &B.pi, &B.omega, &B.F, &B.tau, &B.part }) b->release();
   dev_ewald_release(d);
   dev_structs_release(d);
   if (d->hstage) (void)hipHostFree(d->hstage);
