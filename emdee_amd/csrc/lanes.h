@@ -9,7 +9,7 @@ namespace emdee {
 // entries per lane, so that long lists (water at rc 10 A holds ~700 entries
 // per atom) are spread over many waves.
 // Small systems with long lists go past 16, as long as all blocks are resident
-// at once; a second round of a few blocks costs more than the shorter walks
+// at once; a few blocks left over for later cost more than the shorter walks
 // save.  A CU holds four blocks of the FP64 kernels (103 to 122 registers) and
 // five of the mixed (83 to 91), so 32 lanes reach to 8,192 and 10,240 atoms
 // and 64 to 4,096.  Step times, us, with 16 / 32 / 64 lanes:
@@ -21,7 +21,7 @@ namespace emdee {
 //   122: 44.6 / 44.4 / 45.8; 4,096, 353: 51.5 / 48.7 / 49.6) and more atoms
 //   (8,192, 727: 67.8 / 62.5 / 67.4).
 //   16 lanes: 12,288 LJ atoms, 735: 77.3 / 82.4 / 82.7, mixed 79.9 / 83.8 /
-//   80.6.  Water's FP64 terms hide the second round (12,288 atoms, 721:
+//   80.6.  Water's FP64 terms hide the late blocks (12,288 atoms, 721:
 //   143.1 / 141.8 / 144.8), so several types keep 32 to 16,384 atoms.
 // Below 96 entries 16 and 32 lanes are even (2,000 atoms, 91: 43.2 / 42.5).
 inline int pair_lanes(int N, double entries, bool mixed, bool uniform) {
